@@ -221,10 +221,331 @@ __global__ __launch_bounds__(kAtBlock) void attn_split_kernel(const uint16_t* __
     }
 }
 
+// ---------------------------------------------------------------- many token rows
+// Workgroup (n, y, z): head n, token rows 16 y .. + 15 with both query heads (32 query rows), part z of
+// the slots. The four waves take 32-slot tiles in turn (those in which some row has a valid slot), each
+// with an online softmax of its own, on v_mfma_f32_32x32x16_bf16, transposed: scores^T = K Q^T and
+// out^T += V^T P^T, so that a lane holds one query row's values. The weights stay in the registers
+// they are computed in -- step kk of the second product takes slots 16 kk + 4 h + {0..3, 8..11} from
+// lane half h, for V (transposing LDS reads) alike -- and enter as two bf16 parts, high and low (about
+// 16 significant bits; sums of weights are f32 of the whole weights). K and V tiles are loaded a tile
+// ahead into registers, in whole rows, and pass through the wave's own LDS: no barrier in the loop.
+// The waves' states meet in LDS at the end; with several parts (few rows: the slots are spread over
+// up to 8 workgroups), the parts' in attn_merge_kernel.
+// Bound: a workgroup reads every valid slot's K and V of its head once (1 MB of 1024 slots) through the
+// CU's L1, as long as the 48 MFMAs per tile and wave take. 512 rows
+// (causal, from position 300) 30 us, over all slots 34; 1000 rows 57; 16 rows 12 (a workgroup set per row,
+// as above: 693, 694, 1357, 22).
+constexpr int kArRows = 16;                     // token rows per workgroup
+constexpr int kArQ = kArRows * kGs;             // query rows
+constexpr int kArTile = 32;                     // slots per tile
+constexpr int kArTiles = kTs / kArTile;
+constexpr int kArOStride = kDs + 4;             // LDS row of a wave's state, in floats
+constexpr int kArRec = 4 + kDs;                 // record of a query row: reference, sum, 2 unused, out[256]
+constexpr int kArMaxBlocks = 32;                // row blocks x slot parts of a launch with several parts
+// Weights are exp(score - reference) with a reference at most this far below the row's largest score: out
+// (128 accumulators a lane) is rescaled only when the maximum has grown by more.
+constexpr float kArSlack = 8.0f;
+constexpr int kArMinRows = 6;                   // rows of a call from which this path is used: 12 us up to 16 rows, a
+                                                // workgroup set per row takes 11.7 us at 5 rows, 12.1 at 6, 14.2 at 8
+static_assert((size_t)kNs * kArMaxBlocks * kArQ * kArRec <= kAttnPartFloats, "records fit the scratch");
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef short at_s16x4 __attribute__((ext_vector_type(4)));
+typedef float at_f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // mask rows are 4-byte aligned
+typedef __attribute__((address_space(3))) at_s16x4 at_lds_s16x4;
+
+// A K or V row's 16-byte chunk c lies at c ^ ar_swizzle(row) of its LDS row: sixteen consecutive rows
+// take every value, four rows differ by multiples of four chunks.
+__device__ __forceinline__ int ar_swizzle(int row) { return (row & 3) << 2 | (row >> 2 & 3); }
+
+__global__ __launch_bounds__(kAtBlock) __attribute__((amdgpu_waves_per_eu(1, 1))) void attn_rows_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
+    const float* __restrict__ mask, uint16_t* __restrict__ out, int M, float* __restrict__ part) {
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[4 * kArQ * kArOStride * 4];  // K, V tiles (32 KB a wave); then states
+    __shared__ __attribute__((aligned(1024))) uint8_t ql[kArQ * kDs * 2];
+    __shared__ uint64_t bits[kArRows][kTs / 64];
+    __shared__ float st_m[4][kArQ], st_l[4][kArQ];
+    static_assert(sizeof(smem) >= 4 * 2 * kArTile * kDs * 2, "tiles fit");
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int l32 = lane & 31, hf = lane >> 5;
+    const int n = blockIdx.x, m0 = blockIdx.y * kArRows;
+    const int nt = kArTiles / gridDim.z, u0 = blockIdx.z * nt;  // tiles of this part
+
+    // Tile loads: instruction i moves rows 2 i, 2 i + 1 (512 bytes each). Buffer loads at a tile's offset vo; past
+    // the last tile they read nothing. They are spread over other work: issued together, a tile's 32 hold
+    // the wave for two thousand cycles.
+    uint8_t* kl = smem + wave * (2 * kArTile * kDs * 2);
+    uint8_t* vl = kl + kArTile * kDs * 2;
+    constexpr int kRow = kNs * kDs * 2, kCache = kTs * kRow, kNone = 0x40000000;
+    const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(kc), 0, kCache, 0x00020000);
+    const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(vc), 0, kCache, 0x00020000);
+    const int vo0 = hf * kRow + n * kDs * 2 + 16 * l32;
+    uint4 kr[16], vr[16];
+    auto load_k = [&](int vo, int i) { kr[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(krs, vo, 2 * i * kRow, 0)); };
+    auto load_v = [&](int vo, int i) { vr[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(vrs, vo, 2 * i * kRow, 0)); };
+    auto load_tile = [&](int u) {
+        const int vo = vo0 + (u0 + u) * kArTile * kRow;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) load_k(vo, i);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) load_v(vo, i);
+    };
+    const int guess = min(wave, nt - 1);  // the wave's first tile when all are wanted
+    {
+        // valid slots of rows 4 w .. 4 w + 3 (16 per lane), Q (query row l32: token row l32 / 2, head l32 % 2; wave w
+        // brings rows 8 w .. + 7), then the guessed tile
+        at_f32x4u v[4][4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                v[r][i] = *reinterpret_cast<const at_f32x4u*>(mask + (size_t)min(m0 + 4 * wave + r, M - 1) * kTs + 16 * lane + 4 * i);
+        uint4 qv[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int qr = 8 * wave + 2 * i + hf;
+            qv[i] = ld16(q + (((size_t)min(m0 + qr / kGs, M - 1) * kNs + n) * kGs + qr % kGs) * kDs + 8 * l32);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        load_tile(guess);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            uint32_t b = 0;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) b |= v[r][i >> 2][i & 3] != 0.0f ? 1u << i : 0u;
+            reinterpret_cast<uint16_t*>(bits[4 * wave + r])[lane] = m0 + 4 * wave + r < M ? (uint16_t)b : 0;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int qr = 8 * wave + 2 * i + hf;
+            *reinterpret_cast<uint4*>(ql + qr * 512 + (l32 ^ ar_swizzle(qr)) * 16) = qv[i];
+        }
+    }
+    __syncthreads();
+    uint32_t mine = 0;  // this wave's tiles
+    {
+        uint32_t any = 0;
+        if (lane < nt)
+#pragma unroll
+            for (int r = 0; r < kArRows; ++r) any |= (uint32_t)(bits[r][(u0 + lane) / 2] >> (32 * ((u0 + lane) & 1)));
+        uint32_t todo = (uint32_t)__ballot(any != 0);
+        for (int c = 0; todo; ++c, todo &= todo - 1)
+            if ((c & 3) == wave) mine |= todo & -todo;
+    }
+
+    // LDS addresses: writes (row 2 i + hf: i % 8 here, i / 8 as 16 rows), K reads (chunk 2 j + hf of row l32:
+    // j % 8 here, j / 8 as 256 bytes), V reads (dim tile dt, slots 8 y + 4 hf + (lane % 16) / 4 of step kk)
+    int wa[8], ka[8], va[4];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) wa[i] = (2 * i + hf) * 512 + (l32 ^ ar_swizzle(2 * i + hf)) * 16;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ka[j] = l32 * 512 + ((2 * j + hf) ^ ar_swizzle(l32)) * 16;
+    const int i16 = lane & 15, vrow = 4 * hf + (i16 >> 2), vch = 2 * (lane >> 4 & 1) + (i16 >> 1 & 1);
+    // rows 16 kk + 8 y + vrow: row & 3 = i16 / 4, row >> 2 & 3 = 2 y + hf
+#pragma unroll
+    for (int d = 0; d < 4; ++d) va[d] = vrow * 512 + ((4 * d + vch) ^ ((i16 >> 2) << 2 | hf)) * 16 + (i16 & 1) * 8;
+
+    f32x16 o[8];
+#pragma unroll
+    for (int d = 0; d < 8; ++d)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[d][e] = 0.0f;
+    float m_ref = -INFINITY, l_run = 0.0f;  // the score that the row's weights are relative to, their sum
+    int u = mine ? __builtin_ctz(mine) : 0;
+    if (mine && u != guess) load_tile(u);
+    while (mine) {
+        mine &= mine - 1;
+        const int un = mine ? __builtin_ctz(mine) : 0;
+        const int vo = mine ? vo0 + (u0 + un) * kArTile * kRow : kNone;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) *reinterpret_cast<uint4*>(kl + wa[i & 7] + (i >> 3) * 16 * 512) = kr[i];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) *reinterpret_cast<uint4*>(vl + wa[i & 7] + (i >> 3) * 16 * 512) = vr[i];
+        f32x16 sc[2];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sc[0][e] = sc[1][e] = 0.0f;
+        // four K and Q fragments (both of row l32, same chunk) ahead of the MFMAs, the next tile's K beside them
+        bf16x8 kf[4], qf[4];
+        auto read_k = [&](int j) {
+            kf[j & 3] = *reinterpret_cast<const bf16x8*>(kl + ka[j & 7] + (j >> 3) * 256);
+            qf[j & 3] = *reinterpret_cast<const bf16x8*>(ql + ka[j & 7] + (j >> 3) * 256);
+        };
+#pragma unroll
+        for (int j = 0; j < 4; ++j) read_k(j);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            sc[j & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[j & 3], qf[j & 3], sc[j & 1], 0, 0, 0);
+            if (j < 12) read_k(j + 4);
+            load_k(vo, j);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // element e: slot 8 (e / 4) + 4 hf + e % 4 of the tile
+        const uint32_t vb = (uint32_t)(bits[l32 >> 1][(u0 + u) / 2] >> (32 * ((u0 + u) & 1) + 4 * hf));
+        float mx = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sc[0][e] += sc[1][e];
+        if (!__all((vb & 0x0f0f0f0fu) == 0x0f0f0f0fu)) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) sc[0][e] = (vb >> (8 * (e >> 2) + (e & 3)) & 1) ? sc[0][e] : -INFINITY;
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sc[0][e]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        float scale = 1.0f;
+        if (mx > m_ref + kArSlack) {
+            scale = m_ref == -INFINITY ? 1.0f : __expf(m_ref - mx);  // -inf: sum and out are still zero
+            m_ref = mx;
+        }
+        const float mu = m_ref == -INFINITY ? 0.0f : m_ref;
+        float ls = 0.0f;
+        uint32_t ph[8], pl[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float p0 = __expf(sc[0][2 * i] - mu), p1 = __expf(sc[0][2 * i + 1] - mu);
+            ls += p0;
+            ls += p1;
+            ph[i] = pk_bf16(p0, p1);
+            pl[i] = pk_bf16(p0 - __uint_as_float(ph[i] << 16), p1 - __uint_as_float(ph[i] & 0xffff0000u));
+        }
+        l_run = fmaf(l_run, scale, ls + __shfl_xor(ls, 32));
+        if (__any(scale != 1.0f)) {
+#pragma unroll
+            for (int d = 0; d < 8; ++d)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) o[d][e] *= scale;
+        }
+        // step x: slots 16 (x / 8) .. + 15, dim tile x % 8; V two steps ahead, the next tile's V beside them
+        bf16x8 vf[3];
+        auto read_v = [&](bf16x8& f, int x) {
+            at_s16x4 a[2];
+#pragma unroll
+            for (int y = 0; y < 2; ++y)  // y flips bit 1 of the swizzle: 32 bytes
+                a[y] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (at_lds_s16x4*)(vl + (va[x & 3] ^ (32 * y)) + (16 * (x >> 3) + 8 * y) * 512 + (x >> 2 & 1) * 256));
+            f = __builtin_bit_cast(bf16x8, __builtin_shufflevector(a[0], a[1], 0, 1, 2, 3, 4, 5, 6, 7));
+        };
+        read_v(vf[0], 0);
+        read_v(vf[1], 1);
+#pragma unroll
+        for (int x = 0; x < 16; ++x) {
+            if (x < 14) read_v(vf[(x + 2) % 3], x + 2);
+            load_v(vo, x);
+            const int k = 4 * (x >> 3);
+            o[x & 7] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                vf[x % 3], __builtin_bit_cast(bf16x8, make_uint4(ph[k], ph[k + 1], ph[k + 2], ph[k + 3])), o[x & 7], 0, 0, 0);
+            o[x & 7] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                vf[x % 3], __builtin_bit_cast(bf16x8, make_uint4(pl[k], pl[k + 1], pl[k + 2], pl[k + 3])), o[x & 7], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        u = un;
+    }
+    // the waves' states, brought to the largest reference
+    if (hf == 0) {
+        st_m[wave][l32] = m_ref;
+        st_l[wave][l32] = l_run;
+    }
+    __syncthreads();
+    const float mt = fmaxf(fmaxf(st_m[0][l32], st_m[1][l32]), fmaxf(st_m[2][l32], st_m[3][l32]));
+    const float f = m_ref == -INFINITY ? 0.0f : __expf(m_ref - mt);
+    float* os = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int d = 0; d < 8; ++d)
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+            *reinterpret_cast<float4*>(os + (wave * kArQ + l32) * kArOStride + 32 * d + 8 * a + 4 * hf) =
+                make_float4(o[d][4 * a] * f, o[d][4 * a + 1] * f, o[d][4 * a + 2] * f, o[d][4 * a + 3] * f);
+    __syncthreads();
+    // thread t: query row t / 8, dims 8 (t % 8) + 64 i
+    const int qr = t >> 3, m = m0 + qr / kGs;
+    float mq = -INFINITY, lq = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) mq = fmaxf(mq, st_m[w][qr]);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) lq += st_m[w][qr] == -INFINITY ? 0.0f : st_l[w][qr] * __expf(st_m[w][qr] - mq);
+    if (m >= M) return;
+    float* rec = part + ((((size_t)blockIdx.y * kNs + n) * gridDim.z + blockIdx.z) * kArQ + qr) * kArRec;
+    if (gridDim.z > 1 && (t & 7) == 0) {
+        rec[0] = mq;
+        rec[1] = lq;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int d = 8 * (t & 7) + 64 * i;
+        float v[8];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            float4 a = *reinterpret_cast<const float4*>(os + qr * kArOStride + d + 4 * h);
+#pragma unroll
+            for (int w = 1; w < 4; ++w) {
+                const float4 b = *reinterpret_cast<const float4*>(os + (w * kArQ + qr) * kArOStride + d + 4 * h);
+                a.x += b.x;
+                a.y += b.y;
+                a.z += b.z;
+                a.w += b.w;
+            }
+            v[4 * h] = a.x;
+            v[4 * h + 1] = a.y;
+            v[4 * h + 2] = a.z;
+            v[4 * h + 3] = a.w;
+            if (gridDim.z > 1) *reinterpret_cast<float4*>(rec + 4 + d + 4 * h) = a;
+        }
+        if (gridDim.z == 1) {
+            uint32_t h[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) h[e] = pk_bf16(lq > 0.0f ? v[2 * e] / lq : 0.0f, lq > 0.0f ? v[2 * e + 1] / lq : 0.0f);
+            *reinterpret_cast<uint4*>(out + (((size_t)m * kNs + n) * kGs + qr % kGs) * kDs + d) =
+                make_uint4(h[0], h[1], h[2], h[3]);
+        }
+    }
+}
+
+// Workgroup (n, m): the nz (at most 8) slot parts of token row m, head n; thread t: query head t / 128,
+// dims 2 (t % 128), + 1.
+__global__ __launch_bounds__(kAtBlock) void attn_merge_kernel(const float* __restrict__ part, int nz, uint16_t* __restrict__ out) {
+    const int n = blockIdx.x, m = blockIdx.y, t = threadIdx.x, g = t >> 7, d = 2 * (t & 127);
+    const float* rec = part + ((((size_t)(m / kArRows) * kNs + n) * nz) * kArQ + (m % kArRows) * kGs + g) * kArRec;
+    float mz[8], lz[8], mt = -INFINITY;
+    float2 oz[8];
+#pragma unroll
+    for (int z = 0; z < 8; ++z) {
+        const float* r = rec + (size_t)min(z, nz - 1) * kArQ * kArRec;
+        mz[z] = z < nz ? r[0] : -INFINITY;
+        lz[z] = r[1];
+        oz[z] = *reinterpret_cast<const float2*>(r + 4 + d);
+    }
+#pragma unroll
+    for (int z = 0; z < 8; ++z) mt = fmaxf(mt, mz[z]);
+    float l = 0.0f, a = 0.0f, b = 0.0f;
+#pragma unroll
+    for (int z = 0; z < 8; ++z) {
+        const float f = mz[z] == -INFINITY ? 0.0f : __expf(mz[z] - mt);
+        l = fmaf(f, lz[z], l);
+        a = fmaf(f, oz[z].x, a);
+        b = fmaf(f, oz[z].y, b);
+    }
+    *reinterpret_cast<uint32_t*>(out + (((size_t)m * kNs + n) * kGs + g) * kDs + d) =
+        pk_bf16(l > 0.0f ? a / l : 0.0f, l > 0.0f ? b / l : 0.0f);
+}
+
 }  // namespace
 
 hipError_t launch_sliding_attention(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache, const float* mask,
                                     uint16_t* out, int M, hipStream_t s, DevCtx* ctx) {
+    if (M >= kArMinRows) {
+        // slot parts: as many (1, 2, 4 or 8; a wave needs a tile) as keep the grid within one workgroup per CU
+        const int blocks = (M + kArRows - 1) / kArRows;
+        int nz = 1;
+        while (nz < 8 && blocks * nz * 2 <= kArMaxBlocks) nz *= 2;
+        hipLaunchKernelGGL(attn_rows_kernel, dim3(kNs, blocks, nz), dim3(kAtBlock), 0, s, q, k_cache, v_cache, mask, out, M,
+                           ctx->attn_part);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess || nz == 1) return e;
+        hipLaunchKernelGGL(attn_merge_kernel, dim3(kNs, M), dim3(kAtBlock), 0, s, (const float*)ctx->attn_part, nz, out);
+        return hipGetLastError();
+    }
     for (int m0 = 0; m0 < M; m0 += kMaxDecodeM) {
         const int mm = M - m0 < kMaxDecodeM ? M - m0 : kMaxDecodeM;
         hipLaunchKernelGGL(attn_split_kernel, dim3(kNs, kAtChunks, mm), dim3(kAtBlock), 0, s,
