@@ -570,7 +570,14 @@ int moa_full_project_qkv(const uint16_t* x, const uint8_t* q_weight, const uint8
     if (!ctx) return code;
     QkvParams p{x, q_weight, k_weight, nullptr, q_weight_scale, k_weight_scale, nullptr, ScaleKind::BF16,
                 input_rms_weight, q_rms_weight, k_rms_weight, kv_offset, rope_offset, cos, sin, k_cache, v_cache, q_out};
-    return finish(launch_full_qkv(p, M, static_cast<hipStream_t>(stream), ctx), "full_project_qkv launch");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (M <= kMaxDecodeM) return finish(launch_full_qkv(p, M, s, ctx), "full_project_qkv launch");
+    for (int m0 = 0; m0 < M; m0 += kMaxFullQkvM) {
+        const int e = finish(launch_full_qkv_chunk(p, m0, M - m0 < kMaxFullQkvM ? M - m0 : kMaxFullQkvM, s, ctx),
+                             "full_project_qkv launch");
+        if (e) return e;
+    }
+    return MOA_SUCCESS;
 }
 
 static int full_page(const uint16_t* q, const uint16_t* k, const uint16_t* v, const float* mask, float* running_max,
@@ -623,7 +630,14 @@ int moa_full_attention_output(const uint16_t* x, const float* running_sum, const
     DevCtx* ctx = ctx_or_fail(&code);
     if (!ctx) return code;
     OParams p{x, post_attn_rms_weight, o_weight, o_weight_scale, ScaleKind::BF16, residual, running_sum};
-    return finish(launch_full_o(p, M, static_cast<hipStream_t>(stream), ctx), "full_attention_output launch");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (M <= kMaxDecodeM) return finish(launch_full_o(p, M, s, ctx), "full_attention_output launch");
+    for (int m0 = 0; m0 < M; m0 += kMaxChunkM) {
+        const int e = finish(launch_o_chunk(p, m0, M - m0 < kMaxChunkM ? M - m0 : kMaxChunkM, s, ctx),
+                             "full_attention_output launch");
+        if (e) return e;
+    }
+    return MOA_SUCCESS;
 }
 
 int moa_final_norm_and_logits(const uint16_t* input, const uint16_t* rms_weight, const uint16_t* lm_head_weight,

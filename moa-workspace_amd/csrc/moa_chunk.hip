@@ -517,12 +517,28 @@ __global__ __launch_bounds__(kCkBlock) void chunk_rmsnorm_rows_kernel(const uint
 }
 
 // Row-major bf16 [M][K] -> A tiles (the O-projection's input arrives row-major). One workgroup
-// per row (tile_row); thread t moves 16-byte units t, t + 256, ...
-__global__ __launch_bounds__(kCkBlock) void chunk_tile_rows_kernel(const uint16_t* __restrict__ x, int K,
+// per row (tile_row); thread t moves 16-byte units t, t + 256, ... With Div (full-attention output:
+// the running softmax sums [M][16] of the 512-element heads) each element becomes bf16(x / sum), or
+// zero where the sum is not positive -- as rw_rows_load of the rows path.
+template <bool Div>
+__global__ __launch_bounds__(kCkBlock) void chunk_tile_rows_kernel(const uint16_t* __restrict__ x,
+                                                                   const float* __restrict__ div, int K,
                                                                    uint16_t* __restrict__ out) {
     const int m = tile_row(blockIdx.x, gridDim.x);
-    for (int u = threadIdx.x; u < K / 8; u += kCkBlock)
-        *reinterpret_cast<uint4*>(out + atile_off(m, u * 8, K)) = ld16(x + (size_t)m * K + u * 8);
+    for (int u = threadIdx.x; u < K / 8; u += kCkBlock) {
+        uint4 v = ld16(x + (size_t)m * K + u * 8);
+        if constexpr (Div) {
+            const float d = div[m * kGf + u * 8 / kDf];
+            float f[8];
+            bf16x8_to_f32(v, f);
+            uint32_t h[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                h[e] = pk_bf16(d > 0.0f ? f[2 * e] / d : 0.0f, d > 0.0f ? f[2 * e + 1] / d : 0.0f);
+            v = make_uint4(h[0], h[1], h[2], h[3]);
+        }
+        *reinterpret_cast<uint4*>(out + atile_off(m, u * 8, K)) = v;
+    }
 }
 
 // Per (head, row): raw = bf16((sum of the split-K partials) * s), RMSNorm over the head's 256 raw
@@ -774,15 +790,38 @@ hipError_t launch_qkv_chunk(const QkvParams& p, int m0, int M, hipStream_t s, De
         : ck_launch(chunk_qkv_heads4_kernel<ScaleKind::BF16, 4>, dim3(8, M), s, p, m0, M, part, sp, ctx->err);
 }
 
-// O's A tiles and its split-K GEMM into ctx->fbuf; *sp: the splits
-static hipError_t o_chunk_gemm(const OParams& p, int m0, int M, hipStream_t s, DevCtx* ctx, int* sp) {
-    hipError_t e = ck_launch(chunk_tile_rows_kernel, dim3(M), s, p.x + (size_t)m0 * kQs, kQs, ctx->pbuf);
+// full_project_qkv: the rows once through the GEMM over [Wq; Wk], then the head kernel of the rows
+// path. (Called 16 rows at a time, the rows path reads the weights every 16 rows: QKV and O of 300 rows take
+// 610 us that way, 98 us this way.)
+hipError_t launch_full_qkv_chunk(const QkvParams& p, int m0, int M, hipStream_t s, DevCtx* ctx) {
+    constexpr int N = kQf + kPf;
+    hipError_t e = ck_launch(chunk_rmsnorm_rows_kernel<true>, dim3(M), s, p.x + (size_t)m0 * kH, p.in_rms, ctx->hbuf);
     if (e != hipSuccess) return e;
     GemmArgs g{};
-    g.x = ctx->pbuf; g.M = M; g.N = kH; g.K = kQs;
+    g.x = ctx->hbuf; g.M = M; g.N = N; g.K = kH;
+    g.w[0] = p.qw; g.w[1] = p.kw;
+    g.nseg[0] = 0; g.nseg[1] = kQf; g.nseg[2] = N; g.nsegs = 2;
+    g.yf = ctx->fbuf;
+    const bool narrow = m_tiles(M) == 1;  // as launch_qkv_chunk
+    const int sp = pick_splits(N / (narrow ? kCkOBN : kCkBN) * m_tiles(M), kH / kCkBK, (size_t)M * N);
+    e = narrow ? gemm_partial<FfnFormat::FP8, kCkOBN>(g, sp, p.scale_kind, s) : gemm_partial(g, sp, p.scale_kind, s);
+    if (e != hipSuccess) return e;
+    return launch_full_qkv_heads(p, m0, M, ctx->fbuf, sp, s, ctx);
+}
+
+// O's A tiles and its split-K GEMM into ctx->fbuf; *sp: the splits. With p.div, the full-attention
+// layers' O (8192 inputs, divided by the running sums).
+static hipError_t o_chunk_gemm(const OParams& p, int m0, int M, hipStream_t s, DevCtx* ctx, int* sp) {
+    const int K = p.div ? kQf : kQs;
+    const uint16_t* x = p.x + (size_t)m0 * K;
+    hipError_t e = p.div ? ck_launch(chunk_tile_rows_kernel<true>, dim3(M), s, x, p.div + (size_t)m0 * kGf, K, ctx->pbuf)
+                         : ck_launch(chunk_tile_rows_kernel<false>, dim3(M), s, x, (const float*)nullptr, K, ctx->pbuf);
+    if (e != hipSuccess) return e;
+    GemmArgs g{};
+    g.x = ctx->pbuf; g.M = M; g.N = kH; g.K = K;
     g.w[0] = p.ow; g.nseg[0] = 0; g.nseg[1] = kH; g.nsegs = 1;
     g.yf = ctx->fbuf;
-    *sp = pick_splits(kH / kCkOBN * m_tiles(M), kQs / kCkBK, (size_t)M * kH);
+    *sp = pick_splits(kH / kCkOBN * m_tiles(M), K / kCkBK, (size_t)M * kH);
     return gemm_partial<FfnFormat::FP8, kCkOBN>(g, *sp, p.scale_kind, s);
 }
 

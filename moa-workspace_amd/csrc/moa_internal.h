@@ -16,6 +16,9 @@ constexpr int kMaxDecodeM = 16;
 constexpr int kRowsProjMinM = 3;
 // Rows handled by one call of the MFMA (M > kMaxDecodeM) path; larger calls are tiled by the host.
 constexpr int kMaxChunkM = 1024;
+// The same for full_project_qkv: its 8704 columns of f32 sums per row stay within kChunkPartFloats, and
+// a page holds 512 slots.
+constexpr int kMaxFullQkvM = 512;
 // QKV projection rows (Q | K | V).
 constexpr int kQkvRowsTotal = kQs + 2 * kPs;
 // f32 split-K partial sums of the MFMA path: splits x M x N never exceeds one chunk of QKV columns
@@ -177,7 +180,8 @@ hipError_t launch_full_attention(const uint16_t* q, const uint16_t* k_pages, con
 
 // MFMA path for one chunk of 1..kMaxChunkM token rows starting at row m0 of the call.
 hipError_t launch_qkv_chunk(const QkvParams& p, int m0, int M, hipStream_t s, DevCtx* ctx);
-hipError_t launch_o_chunk(const OParams& p, int m0, int M, hipStream_t s, DevCtx* ctx);
+hipError_t launch_o_chunk(const OParams& p, int m0, int M, hipStream_t s, DevCtx* ctx);  // p.div: full-attention O
+hipError_t launch_full_qkv_chunk(const QkvParams& p, int m0, int M, hipStream_t s, DevCtx* ctx);  // at most kMaxFullQkvM rows
 hipError_t launch_ffn_chunk(const FfnParams& p, int m0, int M, hipStream_t s, DevCtx* ctx);  // every format
 // sliding_attention_output then decoder_feedforward on one residual (o.residual == p.residual)
 hipError_t launch_o_ffn_chunk(const OParams& o, const FfnParams& p, int m0, int M, hipStream_t s, DevCtx* ctx);
@@ -191,6 +195,7 @@ hipError_t launch_rmsnorm_rows(const uint16_t* x, const uint16_t* w, uint16_t* o
 // The row kernels after a split-K contraction of M rows (partials [splits][M][N] f32): the QKV heads
 // (scale, head RMSNorm, RoPE, q_out / ring-cache stores) and the O post (scale, post-RMSNorm, residual).
 hipError_t launch_qkv_heads(const QkvParams& p, int m0, int M, const float* part, int splits, hipStream_t s, DevCtx* ctx);
+hipError_t launch_full_qkv_heads(const QkvParams& p, int m0, int M, const float* part, int splits, hipStream_t s, DevCtx* ctx);
 hipError_t launch_post_rows(const float* part, int splits, int M, const void* scale, ScaleKind sk, const uint16_t* w_post,
                             uint16_t* res, const uint16_t* ls, hipStream_t s);
 // The O post rows with the FFN's pre-norm behind them (splits <= 4): the new residual rows into res,

@@ -798,13 +798,16 @@ hipError_t launch_full_qkv_rows(const QkvParams& p, int m0, int M, hipStream_t s
     a.yf = ctx->fbuf;
     e = rw_proj<kRwQkvKR>(a, s);
     if (e != hipSuccess) return e;
-    const int sp = kH / kRwQkvKR;
+    return launch_full_qkv_heads(p, m0, M, ctx->fbuf, kH / kRwQkvKR, s, ctx);
+}
+
+hipError_t launch_full_qkv_heads(const QkvParams& p, int m0, int M, const float* part, int splits, hipStream_t s, DevCtx* ctx) {
     if (p.scale_kind == ScaleKind::F32)
-        hipLaunchKernelGGL((rows_fqkv_heads_kernel<ScaleKind::F32>), dim3(kGf + 1, M), dim3(256), 0, s, p, m0, M,
-                           (const float*)ctx->fbuf, sp, ctx->err);
+        hipLaunchKernelGGL((rows_fqkv_heads_kernel<ScaleKind::F32>), dim3(kGf + 1, M), dim3(256), 0, s, p, m0, M, part,
+                           splits, ctx->err);
     else
-        hipLaunchKernelGGL((rows_fqkv_heads_kernel<ScaleKind::BF16>), dim3(kGf + 1, M), dim3(256), 0, s, p, m0, M,
-                           (const float*)ctx->fbuf, sp, ctx->err);
+        hipLaunchKernelGGL((rows_fqkv_heads_kernel<ScaleKind::BF16>), dim3(kGf + 1, M), dim3(256), 0, s, p, m0, M, part,
+                           splits, ctx->err);
     return hipGetLastError();
 }
 
