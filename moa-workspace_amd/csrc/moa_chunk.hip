@@ -26,7 +26,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kCkBlock = 256;          // four waves
-constexpr int kCkBM = 256;             // rows per workgroup: wave w takes rows 64 w .. 64 w + 63
+constexpr int kCkBM = 256;             // rows per workgroup of the widest tile (see chunk_gemm_kernel)
 constexpr int kCkBN = 128;             // weight rows per workgroup (GeGLU: 64 up + the same 64 gate)
 constexpr int kCkBK = 64;              // k per pipeline step
 constexpr int kCkWStride = 2 * kCkBK + 16;  // LDS bytes per staged (bf16) weight row: 144 puts 16 rows on distinct banks
@@ -133,10 +133,16 @@ constexpr int kCkNt = 0;
 //   All loads are buffer loads whose per-lane offsets are fixed: the step moves the scalar
 //   offset only. Prefetches past the last step repeat the last step (harmless), so the loop body
 //   has no branches.
-template <Epi E, ScaleKind SK, FfnFormat F = FfnFormat::FP8, int BN = kCkBN>
-__global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(1, 1))) void chunk_gemm_kernel(GemmArgs g) {
+//   Fewer rows: RG row groups of 32 MB rows and CG = 4 / RG column groups of waves; wave (rg, cg) takes
+//   32-column blocks cg, cg + CG, .. (so that a GeGLU wave has up and gate of the same columns). BM = 32
+//   MB RG rows: 256 (RG 4, MB 2), 128 (RG 2, MB 2) or 64 (RG 2, MB 1). pick_bm chooses
+//   and has the figures.
+template <Epi E, ScaleKind SK, FfnFormat F = FfnFormat::FP8, int BN = kCkBN, int BM = kCkBM>
+__global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(BM == 256 ? 1 : 2, BM == 256 ? 1 : 2))) void chunk_gemm_kernel(GemmArgs g) {
     static_assert(BN == 128 || (BN == 64 && E == Epi::F32Partial), "128 weight rows, or 64 for split-K partials");
-    constexpr int NB = BN / 32;   // 32-column blocks per wave
+    constexpr int RG = BM == 256 ? 4 : 2, MB = BM / 32 / RG, CG = 4 / RG;
+    static_assert(BM == 256 || BM == 128 || BM == 64, "row tiles");
+    constexpr int NB = BN / 32 / CG;   // 32-column blocks per wave
     constexpr int RPT = BN / 64;  // staged weight rows per thread
     constexpr bool FP4 = F != FfnFormat::FP8;
     // bytes per weight row and per 64-k step; FP4 block-scale bytes per row and per step
@@ -151,8 +157,9 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
     uint8_t(*ws)[kWsBytes] = reinterpret_cast<uint8_t(*)[kWsBytes]>(smem);
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int hf = lane >> 5, l32 = lane & 31;
-    const int m_blk = blockIdx.y * kCkBM;
-    const int m_wave = m_blk + wave * 64;
+    const int rg = wave / CG, cg = wave % CG;
+    const int m_blk = blockIdx.y * BM;
+    const int m_wave = m_blk + rg * 32 * MB;
     const int kz = g.K / gridDim.z, kbeg = blockIdx.z * kz, nsteps = kz / kCkBK;
 
     // staged weight rows of this thread: tile row r0 (and r0 + 64 when BN = 128), k 16 q .. 16 q + 15 of each step
@@ -189,15 +196,15 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
     const int wdst0 = r0 * kCkWStride + 32 * q, wdst1 = (r0 + 64) * kCkWStride + 32 * q;
 
     const int kst = g.K / kCkBK;  // 64-k steps (A tiles) per row block
-    const int rblks = (min(g.M - m_blk, kCkBM) + 31) >> 5;
+    const int rblks = (min(g.M - m_blk, BM) + 31) >> 5;
     const __amdgpu_buffer_rsrc_t ars = ck_rsrc(g.x + (size_t)(m_blk >> 5) * kst * 2048, (uint32_t)rblks * kst * 4096u);
-    int avo[2];
+    int avo[MB];
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb) avo[mb] = ((wave * 2 + mb) * kst * 2048 + lane * 8) * 2 + (kbeg / kCkBK) * 4096;
+    for (int mb = 0; mb < MB; ++mb) avo[mb] = ((rg * MB + mb) * kst * 2048 + lane * 8) * 2 + (kbeg / kCkBK) * 4096;
 
-    f32x16 acc[2][NB];
+    f32x16 acc[MB][NB];
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
@@ -205,7 +212,7 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
 
     constexpr int WD = 6;  // weight register sets: W(s + 2) is loaded six steps before it is staged
     uint4 wr[WD][2];       // [set][row pair]
-    uint4 ar[3][2][4];     // [set][32-row block][16 bytes]: A(s) in set s mod 3, loaded two steps ahead
+    uint4 ar[3][MB][4];    // [set][32-row block][16 bytes]: A(s) in set s mod 3, loaded two steps ahead
     bf16x8 bb[2][4];       // B fragments: [set][MFMA j]
     const int last = nsteps - 1;
     // FP4: .x, .y the 16 codes, .z the block-scale code
@@ -238,25 +245,25 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
             }
         }
     };
-    auto load_a = [&](uint4 (&dst)[2][4], int s) {
+    auto load_a = [&](uint4 (&dst)[MB][4], int s) {
         const int so = min(s, last) * 4096;
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
+        for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 dst[mb][i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ars, avo[mb] + 1024 * i, so, 0));
     };
     auto read_b = [&](bf16x8 (&dst)[4], int buf, int nb) {
-        const bf16x8* bp = reinterpret_cast<const bf16x8*>(&ws[buf][(32 * nb + l32) * kCkWStride + 64 * hf]);
+        const bf16x8* bp = reinterpret_cast<const bf16x8*>(&ws[buf][(32 * (cg + CG * nb) + l32) * kCkWStride + 64 * hf]);
 #pragma unroll
         for (int j = 0; j < 4; ++j) dst[j] = bp[j];
     };
-    auto mfma8 = [&](const uint4 (&a)[2][4], const bf16x8 (&b)[4], auto NBI) {
+    auto mfma8 = [&](const uint4 (&a)[MB][4], const bf16x8 (&b)[4], auto NBI) {
         constexpr int nb = decltype(NBI)::value;
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
-            for (int mb = 0; mb < 2; ++mb)
+            for (int mb = 0; mb < MB; ++mb)
                 acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a[mb][j]), b[j], acc[mb][nb], 0, 0, 0);
     };
 
@@ -274,10 +281,10 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
     load_w(wr[1], WD + 1);
     __syncthreads();
     read_b(bb[0], 0, 0);
-    auto body4 = [&](auto P, int s) {
+    [[maybe_unused]] auto body4 = [&](auto P, int s) {
         constexpr int c = decltype(P)::value;  // s mod 6
         constexpr int cb = c % 3, nbuf = (c + 1) % 3;
-        const uint4(&a)[2][4] = ar[c % 3];
+        const uint4(&a)[MB][4] = ar[c % 3];
         // Fences fix the issue order: each fragment's LDS reads go out during the previous
         // fragment's eight MFMAs, one or two other instructions after each MFMA (a single wave
         // per SIMD issues them while the MFMA runs); the A prefetch rides with fragment 0, the
@@ -343,31 +350,32 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
         __asm__ volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
     };
-    // BN = 64: two fragments per step. Fragment 0 carries the staging (widenings and LDS writes of
+    // Two fragments per step. Fragment 0 carries the staging (widenings and LDS writes of
     // W(s + 2)) beside fragment 1's LDS reads; fragment 1 the A and weight prefetches and, last of
     // the step's LDS operations, the next step's first fragment -- so lgkmcnt(4) at the barrier
     // still leaves every LDS write of this wave complete.
-    auto body2 = [&](auto P, int s) {
+    constexpr int kMf = 4 * MB;  // MFMAs per fragment
+    [[maybe_unused]] auto body2 = [&](auto P, int s) {
         constexpr int c = decltype(P)::value;  // s mod 6
         constexpr int cb = c % 3, nbuf = (c + 1) % 3;
-        const uint4(&a)[2][4] = ar[c % 3];
+        const uint4(&a)[MB][4] = ar[c % 3];
         constexpr int kDsR = 0x100, kDsW = 0x200, kVmR = 0x020, kValu = 0x002, kMfma = 0x008;
-        constexpr int kWLoads = FP4 ? 2 : 1;
-        constexpr int kWValu = F == FfnFormat::NVFP4 ? 4 : 1;
+        constexpr int kWLoads = (FP4 ? 2 : 1) * RPT;
+        constexpr int kWValu = (F == FfnFormat::NVFP4 ? 4 : 1) * RPT * 8 / kMf;
         read_b(bb[1], cb, 1);
         store_w(wr[(c + 2) % WD], (c + 2) % 3);
         mfma8(a, bb[0], Par<0>{});
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < kMf / 2; ++i) {
             __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(kDsR, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(kDsR, 8 / kMf, 0);
             __builtin_amdgcn_sched_group_barrier(kValu, kWValu, 0);
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < kMf / 2; ++i) {
             __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
             __builtin_amdgcn_sched_group_barrier(kValu, kWValu, 0);
-            __builtin_amdgcn_sched_group_barrier(kDsW, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(kDsW, 8 / kMf, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
         load_a(ar[(c + 2) % 3], s + 2);
@@ -375,14 +383,14 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
         read_b(bb[0], nbuf, 0);
         mfma8(a, bb[1], Par<1>{});
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < kMf / 2; ++i) {
             __builtin_amdgcn_sched_group_barrier(kMfma, 1, 1);
             __builtin_amdgcn_sched_group_barrier(kVmR, 2, 1);
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < kMf / 2; ++i) {
             __builtin_amdgcn_sched_group_barrier(kMfma, 1, 1);
-            __builtin_amdgcn_sched_group_barrier(kDsR, 1, 1);
+            __builtin_amdgcn_sched_group_barrier(kDsR, 8 / kMf, 1);
         }
         __builtin_amdgcn_sched_group_barrier(kVmR, kWLoads, 1);
         __builtin_amdgcn_sched_barrier(0);
@@ -391,9 +399,34 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
         __asm__ volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
     };
+    // One fragment per step: everything rides with its MFMAs; the next step's fragment is read last of
+    // the LDS operations, into the other set.
+    [[maybe_unused]] auto body1 = [&](auto P, int s) {
+        constexpr int c = decltype(P)::value;  // s mod 6
+        constexpr int nbuf = (c + 1) % 3;
+        const uint4(&a)[MB][4] = ar[c % 3];
+        constexpr int kDsR = 0x100, kMfma = 0x008;
+        store_w(wr[(c + 2) % WD], (c + 2) % 3);
+        load_a(ar[(c + 2) % 3], s + 2);
+        load_w(wr[(c + 2) % WD], s + 2 + WD);
+        __builtin_amdgcn_sched_barrier(0);
+        read_b(bb[(c + 1) & 1], nbuf, 0);
+        mfma8(a, bb[c & 1], Par<0>{});
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(kDsR, 1, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        __asm__ volatile("s_waitcnt lgkmcnt(4)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __asm__ volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
     auto body = [&](auto P, int s) {
         if constexpr (NB == 4) body4(P, s);
-        else body2(P, s);
+        else if constexpr (NB == 2) body2(P, s);
+        else body1(P, s);
     };
     int s = 0;
     for (; s + 5 < nsteps; s += 6) {
@@ -415,17 +448,17 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
     // Accumulator element r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4 of the 32-row block,
     // column l % 32 of the 32-column block. A wave whose 64 rows all lie below M stores without
     // per-element tests (a test per element would serialise the 64-128 element computations).
-    const bool full = m_wave + 64 <= g.M;
+    const bool full = m_wave + 32 * MB <= g.M;
     if constexpr (E == Epi::F32Partial) {
-        float* yz = g.yf + (size_t)blockIdx.z * g.M * g.N + blockIdx.x * BN + l32;
+        float* yz = g.yf + (size_t)blockIdx.z * g.M * g.N + blockIdx.x * BN + cg * 32 + l32;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-            for (int mb = 0; mb < 2; ++mb)
+            for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int m = m_wave + 32 * mb + 8 * (r >> 2) + 4 * hf + (r & 3);
-                    if (full || m < g.M) yz[(size_t)m * g.N + nb * 32] = acc[mb][nb][r];
+                    if (full || m < g.M) yz[(size_t)m * g.N + CG * nb * 32] = acc[mb][nb][r];
                 }
     } else {
         // p = bf16(gelu(gate) * up) for the wave's 64 rows x 64 columns, transposed through the
@@ -436,37 +469,38 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
         // MXFP4 bf16(sum) (generate_references.py:265-274, 358-372)
         const float gu = F == FfnFormat::NVFP4 ? *g.g0 : 1.0f, gg = F == FfnFormat::NVFP4 ? *g.g2 : 1.0f;
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-            const int n = blockIdx.x * 64 + nb * 32 + l32;
+        for (int nb = 0; nb < NB / 2; ++nb) {
+            const int n = blockIdx.x * 64 + (cg + nb) * 32 + l32;
             const float su = FP4 ? 1.0f : chunk_scale<SK>(g.s0, n), sg = FP4 ? 1.0f : chunk_scale<SK>(g.s2, n);
 #pragma unroll
-            for (int mb = 0; mb < 2; ++mb)
+            for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int ml = 32 * mb + 8 * (r >> 2) + 4 * hf + (r & 3);
                     float up, gate;
                     if constexpr (F == FfnFormat::FP8) {
                         up = rbf(acc[mb][nb][r] * su);
-                        gate = rbf(acc[mb][nb + 2][r] * sg);
+                        gate = rbf(acc[mb][nb + NB / 2][r] * sg);
                     } else if constexpr (F == FfnFormat::NVFP4) {
                         up = rbf(rbf(acc[mb][nb][r]) * gu);
-                        gate = rbf(rbf(acc[mb][nb + 2][r]) * gg);
+                        gate = rbf(rbf(acc[mb][nb + NB / 2][r]) * gg);
                     } else {
                         up = rbf(acc[mb][nb][r]);
-                        gate = rbf(acc[mb][nb + 2][r]);
+                        gate = rbf(acc[mb][nb + NB / 2][r]);
                     }
                     tp[ml * kTpStride + nb * 32 + l32] = (uint16_t)f2bf(rbf(gelu_tanh(gate)) * up);  // gemma4.py:197
                 }
         }
         __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's LDS writes are done
         __builtin_amdgcn_wave_barrier();
-        // 64 rows x 8 units of 16 bytes = 512 units; lane takes units lane + 64 i
+        // 32 MB rows x 64 / CG columns in units of 16 bytes; lane takes units lane + 64 i
+        constexpr int kU = 8 / CG;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int u = lane + 64 * i, ml = u >> 3, cu = u & 7;
+        for (int i = 0; i < MB * kU / 2; ++i) {
+            const int u = lane + 64 * i, ml = u / kU, cu = u % kU;
             const int m = m_wave + ml;
             const uint4 v = *reinterpret_cast<const uint4*>(&tp[ml * kTpStride + cu * 8]);
-            if (full || m < g.M) *reinterpret_cast<uint4*>(g.y + atile_off(m, blockIdx.x * 64 + cu * 8, g.N)) = v;
+            if (full || m < g.M) *reinterpret_cast<uint4*>(g.y + atile_off(m, blockIdx.x * 64 + cg * 32 + cu * 8, g.N)) = v;
         }
     }
 }
@@ -728,25 +762,39 @@ int pick_splits(int tiles, int ksteps, size_t rows_x_cols) {
 // 7.1 us saved in its post rows).
 constexpr int kCkOBN = 64;
 
+// Rows per workgroup of a call of M rows: the smallest row tile that holds them, so that no wave computes
+// rows the call does not have. Past 128 rows, 256: half the widening and weight reads per row. FP8
+// layer (QKV, O, FFN) with 64- / 128- / 256-row tiles: 17 rows 89 / 103 / 120 us, 64 rows 99 / 110 / 126, 128
+// rows 137 / 123 / 138, 200 rows 212 / 176 / 154, 300 rows 290 / 240 / 241, 1000 rows 659 / 543 / 468.
+int pick_bm(int M) { return M <= 64 ? 64 : (M <= 128 ? 128 : kCkBM); }
+
+int m_tiles(int M, int bm) { return (M + bm - 1) / bm; }
+
+template <Epi E, ScaleKind SK, FfnFormat F, int BN>
+hipError_t gemm_launch(const GemmArgs& g, int splits, int bm, hipStream_t s) {
+    const dim3 grid(g.N / (E == Epi::GeGLU ? 64 : BN), m_tiles(g.M, bm), splits);
+    switch (bm) {
+        case 64: return ck_launch(chunk_gemm_kernel<E, SK, F, BN, 64>, grid, s, g);
+        case 128: return ck_launch(chunk_gemm_kernel<E, SK, F, BN, 128>, grid, s, g);
+        case kCkBM: return ck_launch(chunk_gemm_kernel<E, SK, F, BN, kCkBM>, grid, s, g);
+    }
+    return hipErrorInvalidValue;
+}
+
+// Split-K partial sums (the scales are applied by the row kernels that add them).
 template <FfnFormat F = FfnFormat::FP8, int BN = kCkBN>
-hipError_t gemm_partial(const GemmArgs& g, int splits, ScaleKind sk, hipStream_t s) {
+hipError_t gemm_partial(const GemmArgs& g, int splits, int bm, hipStream_t s) {
     if (g.N % BN || g.K % (kCkBK * splits) || (size_t)splits * g.M * g.N > kChunkPartFloats) return hipErrorInvalidValue;
-    const dim3 grid(g.N / BN, (g.M + kCkBM - 1) / kCkBM, splits);
-    if constexpr (F != FfnFormat::FP8) return ck_launch(chunk_gemm_kernel<Epi::F32Partial, ScaleKind::F32, F, BN>, grid, s, g);
-    return sk == ScaleKind::F32 ? ck_launch(chunk_gemm_kernel<Epi::F32Partial, ScaleKind::F32, F, BN>, grid, s, g)
-                                : ck_launch(chunk_gemm_kernel<Epi::F32Partial, ScaleKind::BF16, F, BN>, grid, s, g);
+    return gemm_launch<Epi::F32Partial, ScaleKind::F32, F, BN>(g, splits, bm, s);
 }
 
 template <FfnFormat F = FfnFormat::FP8>
-hipError_t gemm_geglu(const GemmArgs& g, ScaleKind sk, hipStream_t s) {
+hipError_t gemm_geglu(const GemmArgs& g, ScaleKind sk, int bm, hipStream_t s) {
     if (g.N % 64 || g.K % kCkBK) return hipErrorInvalidValue;
-    const dim3 grid(g.N / 64, (g.M + kCkBM - 1) / kCkBM, 1);
-    if constexpr (F != FfnFormat::FP8) return ck_launch(chunk_gemm_kernel<Epi::GeGLU, ScaleKind::F32, F>, grid, s, g);
-    return sk == ScaleKind::F32 ? ck_launch(chunk_gemm_kernel<Epi::GeGLU, ScaleKind::F32>, grid, s, g)
-                                : ck_launch(chunk_gemm_kernel<Epi::GeGLU, ScaleKind::BF16>, grid, s, g);
+    if constexpr (F == FfnFormat::FP8)  // the FP4 formats have no row scales
+        if (sk == ScaleKind::BF16) return gemm_launch<Epi::GeGLU, ScaleKind::BF16, F, kCkBN>(g, 1, bm, s);
+    return gemm_launch<Epi::GeGLU, ScaleKind::F32, F, kCkBN>(g, 1, bm, s);
 }
-
-int m_tiles(int M) { return (M + kCkBM - 1) / kCkBM; }
 
 template <ScaleKind SK>
 hipError_t post_rows(const float* part, int splits, int M, const void* scale, const uint16_t* w_post, uint16_t* res,
@@ -770,10 +818,10 @@ hipError_t launch_qkv_chunk(const QkvParams& p, int m0, int M, hipStream_t s, De
     // Up to 256 rows, 64-row weight tiles (128 tiles x 2 k splits instead of 64 x 4: half the
     // partial sums; M = 256: 39.3 -> 37.4 us). Beyond, they would not split, and the 512 tiles
     // of M = 1024 measured 112 us against 102 with 128-row tiles.
-    const bool narrow = m_tiles(M) == 1;
-    const int sp = pick_splits(kQkvRowsTotal / (narrow ? kCkOBN : kCkBN) * m_tiles(M), kH / kCkBK,
-                               (size_t)M * kQkvRowsTotal);
-    e = narrow ? gemm_partial<FfnFormat::FP8, kCkOBN>(g, sp, p.scale_kind, s) : gemm_partial(g, sp, p.scale_kind, s);
+    const int bm = pick_bm(M), mt = m_tiles(M, bm);
+    const bool narrow = M <= 256;
+    const int sp = pick_splits(kQkvRowsTotal / (narrow ? kCkOBN : kCkBN) * mt, kH / kCkBK, (size_t)M * kQkvRowsTotal);
+    e = narrow ? gemm_partial<FfnFormat::FP8, kCkOBN>(g, sp, bm, s) : gemm_partial(g, sp, bm, s);
     if (e != hipSuccess) return e;
     const float* part = ctx->fbuf;
     if (sp > 4) return hipErrorInvalidValue;  // 60 k steps: pick_splits never gives 8
@@ -802,9 +850,10 @@ hipError_t launch_full_qkv_chunk(const QkvParams& p, int m0, int M, hipStream_t 
     g.w[0] = p.qw; g.w[1] = p.kw;
     g.nseg[0] = 0; g.nseg[1] = kQf; g.nseg[2] = N; g.nsegs = 2;
     g.yf = ctx->fbuf;
-    const bool narrow = m_tiles(M) == 1;  // as launch_qkv_chunk
-    const int sp = pick_splits(N / (narrow ? kCkOBN : kCkBN) * m_tiles(M), kH / kCkBK, (size_t)M * N);
-    e = narrow ? gemm_partial<FfnFormat::FP8, kCkOBN>(g, sp, p.scale_kind, s) : gemm_partial(g, sp, p.scale_kind, s);
+    const int bm = pick_bm(M), mt = m_tiles(M, bm);
+    const bool narrow = M <= 256;  // as launch_qkv_chunk
+    const int sp = pick_splits(N / (narrow ? kCkOBN : kCkBN) * mt, kH / kCkBK, (size_t)M * N);
+    e = narrow ? gemm_partial<FfnFormat::FP8, kCkOBN>(g, sp, bm, s) : gemm_partial(g, sp, bm, s);
     if (e != hipSuccess) return e;
     return launch_full_qkv_heads(p, m0, M, ctx->fbuf, sp, s, ctx);
 }
@@ -821,8 +870,9 @@ static hipError_t o_chunk_gemm(const OParams& p, int m0, int M, hipStream_t s, D
     g.x = ctx->pbuf; g.M = M; g.N = kH; g.K = K;
     g.w[0] = p.ow; g.nseg[0] = 0; g.nseg[1] = kH; g.nsegs = 1;
     g.yf = ctx->fbuf;
-    *sp = pick_splits(kH / kCkOBN * m_tiles(M), K / kCkBK, (size_t)M * kH);
-    return gemm_partial<FfnFormat::FP8, kCkOBN>(g, *sp, p.scale_kind, s);
+    const int bm = pick_bm(M);
+    *sp = pick_splits(kH / kCkOBN * m_tiles(M, bm), K / kCkBK, (size_t)M * kH);
+    return gemm_partial<FfnFormat::FP8, kCkOBN>(g, *sp, bm, s);
 }
 
 hipError_t launch_o_chunk(const OParams& p, int m0, int M, hipStream_t s, DevCtx* ctx) {
@@ -847,15 +897,16 @@ hipError_t ffn_chunk(const FfnParams& p, int m0, int M, hipStream_t s, DevCtx* c
     g.w[0] = p.up; g.w2 = p.gate; g.s0 = p.up_s; g.s2 = p.gate_s;
     g.wsc[0] = (const uint8_t*)p.up_s; g.wsc2 = (const uint8_t*)p.gate_s; g.g0 = p.up_g; g.g2 = p.gate_g;
     g.y = ctx->pbuf;
-    e = gemm_geglu<F>(g, p.scale_kind, s);
+    const int bm = pick_bm(M);
+    e = gemm_geglu<F>(g, p.scale_kind, bm, s);
     if (e != hipSuccess) return e;
     GemmArgs d{};
     d.x = ctx->pbuf; d.M = M; d.N = kH; d.K = kL;
     d.w[0] = p.down; d.nseg[0] = 0; d.nseg[1] = kH; d.nsegs = 1;
     d.wsc[0] = (const uint8_t*)p.down_s;
     d.yf = ctx->fbuf;
-    const int sp = pick_splits(kH / kCkBN * m_tiles(M), kL / kCkBK, (size_t)M * kH);
-    e = gemm_partial<F>(d, sp, p.scale_kind, s);
+    const int sp = pick_splits(kH / kCkBN * m_tiles(M, bm), kL / kCkBK, (size_t)M * kH);
+    e = gemm_partial<F>(d, sp, bm, s);
     if (e != hipSuccess) return e;
     return launch_ffn_post_rows(p, ctx->fbuf, sp, M, res, s);
 }
