@@ -32,6 +32,7 @@ constexpr int kCkBK = 64;              // k per pipeline step
 constexpr int kCkWStride = 2 * kCkBK + 16;  // LDS bytes per staged (bf16) weight row: 144 puts 16 rows on distinct banks
 constexpr int kCkTilesTarget = 264;    // split-K aims at about one workgroup per CU
 constexpr int kCkSplitMax = 8;
+constexpr int kCkHeadRows = 2;         // rows per wave of the QKV heads kernel
 
 // 8 E4M3 codes (two dwords, lower index in the low byte) widened to 8 bf16.
 __device__ __forceinline__ bf16x8 fp8x8_to_bf16(uint32_t lo, uint32_t hi) {
@@ -630,69 +631,85 @@ __global__ __launch_bounds__(kCkBlock) void chunk_qkv_heads_kernel(QkvParams p, 
     dst[t] = (uint16_t)f2bf(a + b);
 }
 
-// The same per (head, row) work for the MFMA path, four heads of one row per workgroup: wave w
-// takes head 4 x + w of row y (x = blockIdx.x < 8, so the four are all Q, all K or all V), lane l
-// its elements l, l + 64, l + 128 and l + 192. Both RoPE pairs (t, t ^ 128) are then within the
-// lane, and the head's sum of squares is four wave sums added in the order of ck_block_sum (wave k
-// there holds elements 64 k ..), so every output has chunk_qkv_heads_kernel's bits; no LDS and no
-// barrier. 8 x M workgroups instead of 32 x M.
-template <ScaleKind SK, int ZS>
-__global__ __launch_bounds__(kCkBlock) void chunk_qkv_heads4_kernel(QkvParams p, int m0, int M,
-                                                                    const float* __restrict__ part, int splits,
-                                                                    uint32_t* err) {
-    const int lane = threadIdx.x & 63, head = 4 * blockIdx.x + (threadIdx.x >> 6), m = blockIdx.y;
+// The same per (head, row) work for the MFMA path: wave w of workgroup (x, y) takes head 4 x + w (x =
+// blockIdx.x < 8, so the four are all Q, all K or all V) of rows RP y .. + RP - 1, lane l its elements
+// 4 l .. 4 l + 3. RoPE partners (t, t ^ 128) are 32 lanes apart: no LDS, no barrier. Bound by the read of
+// the partial sums: all loads of the RP rows, 16 bytes per lane, go out before any is used, and the
+// head's weights and scales are read once for them. 1000 rows
+// (33 MB of sums) 16 us, 256 rows (17 MB) 8; with a lane's four elements 64 apart in 4-byte loads, one row
+// per wave, 32 and 11.
+template <ScaleKind SK, int ZS, int RP>
+__global__ __launch_bounds__(kCkBlock) void chunk_qkv_head_rows_kernel(QkvParams p, int m0, int M,
+                                                                       const float* __restrict__ part, uint32_t* err) {
+    const int lane = threadIdx.x & 63, head = 4 * blockIdx.x + (threadIdx.x >> 6), mr = blockIdx.y * RP;
+    const int col = head * kDs + 4 * lane;
+    float4 pz[RP][ZS];
+#pragma unroll
+    for (int i = 0; i < RP; ++i)
+#pragma unroll
+        for (int z = 0; z < ZS; ++z)
+            pz[i][z] = *reinterpret_cast<const float4*>(part + ((size_t)z * M + min(mr + i, M - 1)) * kQkvRowsTotal + col);
     const int32_t rope_off = *p.rope_off, kv_off = *p.kv_off;
-    const int mm = m0 + m;
-    const bool rope_ok = rope_off >= 0 && (rope_off % (kDs * 2)) == 0 && rope_off / (kDs * 2) + mm < kE;
+    const bool rope_al = rope_off >= 0 && (rope_off % (kDs * 2)) == 0;
     const bool kv_ok = kv_off >= 0 && (kv_off % (kNs * kDs * 2)) == 0 && kv_off / (kNs * kDs * 2) < kTs;
-    if (!rope_ok || !kv_ok) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(err, (rope_ok ? 0u : kErrRopeOffset) | (kv_ok ? 0u : kErrKvOffset));
-        return;
-    }
-    const int slot = (kv_off / (kNs * kDs * 2) + mm) % kTs;
-    const int trow = rope_off / (kDs * 2) + mm;
-    const float* prow = part + (size_t)m * kQkvRowsTotal + head * kDs + lane;
-    float pz[4][ZS];  // all partial loads in flight at once (split index clamped)
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-        for (int z = 0; z < ZS; ++z) pz[k][z] = prow[(size_t)min(z, splits - 1) * M * kQkvRowsTotal + 64 * k];
+    const int trow0 = rope_off / (kDs * 2) + m0, slot0 = kv_off / (kNs * kDs * 2) + m0;
     const uint16_t* wn = head < 16 ? p.q_rms : (head < 24 ? p.k_rms : nullptr);
-    float v[4], ss[4];
+    const void* scp = head < 16 ? p.qs : (head < 24 ? p.ks : p.vs);
+    const int c0 = head < 16 ? 0 : (head < 24 ? kQs : kQs + kPs);
+    float sc[4], wv[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int col = head * kDs + 64 * k + lane;
-        float acc = pz[k][0];
-#pragma unroll
-        for (int z = 1; z < ZS; ++z) acc = z < splits ? acc + pz[k][z] : acc;
-        const float sc = head < 16 ? chunk_scale<SK>(p.qs, col)
-                                   : (head < 24 ? chunk_scale<SK>(p.ks, col - kQs) : chunk_scale<SK>(p.vs, col - kQs - kPs));
-        v[k] = rbf(acc * sc);
-        ss[k] = wave_sum(v[k] * v[k]);
+    for (int e = 0; e < 4; ++e) {
+        sc[e] = chunk_scale<SK>(scp, col - c0 + e);
+        wv[e] = wn ? bf2f(wn[4 * lane + e]) : 1.0f;
     }
-    const float inv = rms_inverse(((ss[0] + ss[1]) + ss[2]) + ss[3], kDs);
-    float n[4];
+    uint2 cq[RP], sq[RP];
+    bool ok[RP];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        float x = v[k] * inv;
-        if (wn) x = x * bf2f(wn[64 * k + lane]);
-        n[k] = rbf(x);
+    for (int i = 0; i < RP; ++i) {
+        const bool rope_ok = rope_al && trow0 + mr + i < kE;
+        ok[i] = mr + i < M && rope_ok && kv_ok;
+        const size_t at = (size_t)(ok[i] ? trow0 + mr + i : 0) * kDs + 4 * lane;
+        cq[i] = *reinterpret_cast<const uint2*>(p.cos + at);
+        sq[i] = *reinterpret_cast<const uint2*>(p.sin + at);
+        if (mr + i < M && !ok[i] && head == 0 && lane == 0)
+            atomicOr(err, (rope_ok ? 0u : kErrRopeOffset) | (kv_ok ? 0u : kErrKvOffset));
     }
-    if (head >= 24) {
-        uint16_t* vd = p.v_cache + (size_t)slot * (kNs * kDs) + (head - 24) * kDs + lane;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) vd[64 * k] = (uint16_t)f2bf(n[k]);
-        return;
-    }
-    // the table's sin has its low half negated (generate_references.py:200-210): plain half swap
-    uint16_t* dst = (head < 16 ? p.q_out + (size_t)mm * kQs + head * kDs
-                               : p.k_cache + (size_t)slot * (kNs * kDs) + (head - 16) * kDs) + lane;
+    for (int i = 0; i < RP; ++i) {
+        float a[4] = {pz[i][0].x, pz[i][0].y, pz[i][0].z, pz[i][0].w};
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int t = 64 * k + lane;
-        const float cv = bf2f(p.cos[(size_t)trow * kDs + t]);
-        const float sv = bf2f(p.sin[(size_t)trow * kDs + t]);
-        dst[64 * k] = (uint16_t)f2bf(rbf(n[k] * cv) + rbf(n[k ^ 2] * sv));
+        for (int z = 1; z < ZS; ++z) {
+            a[0] += pz[i][z].x;
+            a[1] += pz[i][z].y;
+            a[2] += pz[i][z].z;
+            a[3] += pz[i][z].w;
+        }
+        float ss = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            a[e] = rbf(a[e] * sc[e]);
+            ss = fmaf(a[e], a[e], ss);
+        }
+        const float inv = rms_inverse(wave_sum(ss), kDs);
+        float n[4], o[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float x = a[e] * inv;
+            if (wn) x = x * wv[e];
+            n[e] = rbf(x);
+        }
+        const uint32_t cw[2] = {cq[i].x, cq[i].y}, sw[2] = {sq[i].x, sq[i].y};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            // the table's sin has its low half negated (generate_references.py:200-210): plain half swap
+            const float c = bf2f(cw[e >> 1] >> (16 * (e & 1)) & 0xffffu), sn = bf2f(sw[e >> 1] >> (16 * (e & 1)) & 0xffffu);
+            o[e] = head < 24 ? rbf(n[e] * c) + rbf(__shfl_xor(n[e], 32) * sn) : n[e];
+        }
+        if (!ok[i]) continue;
+        const int slot = (slot0 + mr + i) % kTs;
+        uint16_t* dst = head < 16 ? p.q_out + (size_t)(m0 + mr + i) * kQs + head * kDs
+                                  : (head < 24 ? p.k_cache : p.v_cache) + (size_t)slot * (kNs * kDs) + (head & 7) * kDs;
+        *reinterpret_cast<uint2*>(dst + 4 * lane) = make_uint2(pk_bf16(o[0], o[1]), pk_bf16(o[2], o[3]));
     }
 }
 
@@ -807,6 +824,18 @@ hipError_t post_rows(const float* part, int splits, int M, const void* scale, co
 
 }  // namespace
 
+template <ScaleKind SK>
+static hipError_t qkv_head_rows(const QkvParams& p, int m0, int M, const float* part, int splits, hipStream_t s, DevCtx* ctx) {
+    constexpr int RP = kCkHeadRows;
+    const dim3 grid(8, (M + RP - 1) / RP);
+    switch (splits) {  // 60 k steps: pick_splits gives 1, 2 or 4
+        case 1: return ck_launch(chunk_qkv_head_rows_kernel<SK, 1, RP>, grid, s, p, m0, M, part, ctx->err);
+        case 2: return ck_launch(chunk_qkv_head_rows_kernel<SK, 2, RP>, grid, s, p, m0, M, part, ctx->err);
+        case 4: return ck_launch(chunk_qkv_head_rows_kernel<SK, 4, RP>, grid, s, p, m0, M, part, ctx->err);
+    }
+    return hipErrorInvalidValue;
+}
+
 hipError_t launch_qkv_chunk(const QkvParams& p, int m0, int M, hipStream_t s, DevCtx* ctx) {
     hipError_t e = ck_launch(chunk_rmsnorm_rows_kernel<true>, dim3(M), s, p.x + (size_t)m0 * kH, p.in_rms, ctx->hbuf);
     if (e != hipSuccess) return e;
@@ -823,19 +852,8 @@ hipError_t launch_qkv_chunk(const QkvParams& p, int m0, int M, hipStream_t s, De
     const int sp = pick_splits(kQkvRowsTotal / (narrow ? kCkOBN : kCkBN) * mt, kH / kCkBK, (size_t)M * kQkvRowsTotal);
     e = narrow ? gemm_partial<FfnFormat::FP8, kCkOBN>(g, sp, bm, s) : gemm_partial(g, sp, bm, s);
     if (e != hipSuccess) return e;
-    const float* part = ctx->fbuf;
-    if (sp > 4) return hipErrorInvalidValue;  // 60 k steps: pick_splits never gives 8
-    // Up to 256 rows, one workgroup per (head, row): more workgroups hide the loads better (four
-    // heads per workgroup measured 28.5 -> 30.6 us for the call at M = 100, even at 256); beyond,
-    // four heads per workgroup (M = 1024: 101.5 -> 94.1 us).
-    if (narrow) return launch_qkv_heads(p, m0, M, part, sp, s, ctx);
-    if (sp <= 2)  // as many partial loads in flight as there are splits
-        return p.scale_kind == ScaleKind::F32
-            ? ck_launch(chunk_qkv_heads4_kernel<ScaleKind::F32, 2>, dim3(8, M), s, p, m0, M, part, sp, ctx->err)
-            : ck_launch(chunk_qkv_heads4_kernel<ScaleKind::BF16, 2>, dim3(8, M), s, p, m0, M, part, sp, ctx->err);
-    return p.scale_kind == ScaleKind::F32
-        ? ck_launch(chunk_qkv_heads4_kernel<ScaleKind::F32, 4>, dim3(8, M), s, p, m0, M, part, sp, ctx->err)
-        : ck_launch(chunk_qkv_heads4_kernel<ScaleKind::BF16, 4>, dim3(8, M), s, p, m0, M, part, sp, ctx->err);
+    return p.scale_kind == ScaleKind::F32 ? qkv_head_rows<ScaleKind::F32>(p, m0, M, ctx->fbuf, sp, s, ctx)
+                                          : qkv_head_rows<ScaleKind::BF16>(p, m0, M, ctx->fbuf, sp, s, ctx);
 }
 
 // full_project_qkv: the rows once through the GEMM over [Wq; Wk], then the head kernel of the rows
