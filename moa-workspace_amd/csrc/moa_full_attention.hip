@@ -365,19 +365,311 @@ __global__ __launch_bounds__(kFaBlock) void fattn_span_kernel(const uint16_t* __
         for (int r = 0; r < 4; ++r) pc[2 * kGf + (4 * g + r) * kDf + 128 * wave + 16 * dd + l16] = o[dd][r];
 }
 
-// Workgroup (h, m) merges head h's 8 chunk partials into the row's state; thread t owns dims
+// Several token rows: all their heads share the one KV head, so a tile of 64 slots is read once for
+// four rows (64 query rows of 512). Workgroup (x, y): rows 4 y .. 4 y + 3, tiles x * tpw .. (64
+// slots; a page holds 8), an online softmax over those of its tiles in which some row has a valid
+// slot; record x of each row. On v_mfma_f32_32x32x16_bf16, transposed, so that a lane holds one
+// query row's values:
+//   scores^T = K Q^T: wave (sh, qh) takes 32 of the slots and 32 of the query rows, whose 512 dims stay in
+//     registers; the two slot halves exchange their maxima through LDS, sums stay apart to the end;
+//   out^T += V^T P^T: wave w takes dims 128 w .. + 127 of all 64 query rows, over the weights of both
+//     slot halves from LDS (bf16 high and low parts, as in the kernels above).
+// K and V tiles go straight to LDS (16-byte chunks of a row permuted by fr_swizzle, so that neither
+// the K rows' reads nor V's transposing reads meet on banks): the next tile's K while the
+// weights and out are computed, its V while its scores are. 96 MFMAs a tile and wave.
+constexpr int kFrRows = 4;                      // token rows per workgroup
+constexpr int kFrQ = kFrRows * kGf;             // query rows
+constexpr int kFrMaxTiles = 64;                 // tiles per workgroup
+constexpr int kFrPStride = kFaChunk + 8;        // LDS row of the weights, in elements
+// Weights are exp(score - reference) with a reference at most this far below the row's largest score: out
+// (128 accumulators a lane) is rescaled only when the maximum has grown by more, which after the
+// first tile it hardly does, not at every new maximum. The state is brought to the maximum at the end.
+constexpr float kFrSlack = 8.0f;
+// From these row x pages products of a call over all pages (rows of a one-page call) on this path is used.
+// All pages, this path against the one-row kernels on every row: M x P = 2 x 8 18.2 / 15.8 us, 4 x 3 19.0 /
+// 15.2, 16 x 1 19.8 / 16.2, 3 x 8 21.0 / 21.4, 13 x 3 23.7 / 34.0, 2 x 64 29.1 / 37.3, 200 x 6 66 / 840.
+// One page: 16 rows 18.4 / 15.1 us; more would be several launches of the one-row kernel (64 rows 25.6 / 59.2).
+constexpr int kFrMinRowPages = 24;
+constexpr int kFrMinPageRows = 17;
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef short fa_s16x4 __attribute__((ext_vector_type(4)));
+typedef float fa_f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // mask rows are 4-byte aligned
+typedef __attribute__((address_space(3))) fa_s16x4 fa_lds_s16x4;
+
+// The chunk of a K or V row in which its 16-byte chunk c lies in LDS: c ^ fr_swizzle(row). Sixteen
+// consecutive rows take every value, four rows differ by multiples of four chunks.
+__host__ __device__ constexpr int fr_swizzle(int row) { return (row & 3) << 2 | (row >> 2 & 3); }
+
+// LDS barrier that leaves global loads in flight (loads into LDS are waited for explicitly).
+__device__ __forceinline__ void fr_barrier() {
+    __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __asm__ volatile("" ::: "memory");
+}
+
+__global__ __launch_bounds__(kFaBlock) __attribute__((amdgpu_waves_per_eu(1, 1))) void fattn_rows_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
+    const float* __restrict__ mask, int mask_page_stride, int M, int ntiles, int tpw, float* part) {
+    __shared__ __attribute__((aligned(1024))) uint16_t ks[kFaChunk * kDf];
+    __shared__ __attribute__((aligned(1024))) uint16_t vs[kFaChunk * kDf];
+    __shared__ __attribute__((aligned(16))) uint16_t ps[2][kFrQ * kFrPStride];
+    __shared__ uint64_t bits[kFrRows][kFrMaxTiles];   // bit s: slot s of the tile is valid for the row
+    __shared__ float red[2][kFrQ], scl[kFrQ];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l32 = lane & 31, hf = lane >> 5;
+    const int m0 = blockIdx.y * kFrRows;
+    const int u0 = blockIdx.x * tpw, nt = min(tpw, ntiles - u0);
+    const int sh = wave & 1, qh = wave >> 1;
+
+    // K or V tile u into LDS: wave w moves rows 16 w .. 16 w + 15, a row (1 KB) per instruction
+    const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(kc + (size_t)u0 * kFaChunk * kDf), 0, (uint32_t)nt * kFaChunk * kDf * 2, 0x00020000);
+    const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(vc + (size_t)u0 * kFaChunk * kDf), 0, (uint32_t)nt * kFaChunk * kDf * 2, 0x00020000);
+    // (rows i0 .. i1 - 1 of the wave's 16; the loads are spread over other work: issued together they hold the
+    // wave for a thousand cycles)
+    auto issue = [&](__amdgpu_buffer_rsrc_t rs, uint16_t* dst, int u, int i0, int i1) {
+        int ln = lane;
+        __asm__ volatile("" : "+v"(ln));  // the 16 permuted offsets are made anew: kept, they would not fit the registers
+#pragma unroll
+        for (int i = i0; i < i1; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (fa_lds_void*)(dst + (wave * 16 + i) * kDf), 16,
+                                                     (ln ^ fr_swizzle(i)) * 16, (u * kFaChunk + wave * 16 + i) * kDf * 2, 0, 0);
+    };
+    issue(krs, ks, 0, 0, 16);  // most often the first tile it needs (else read again)
+    // Q: lane (l32, hf) holds query row 32 qh + l32, dims 16 j + 8 hf .. + 7 (a row past M repeats the last)
+    uint4 qf[32];
+    {
+        const int qr = 32 * qh + l32;
+        const uint16_t* qp = q + ((size_t)min(m0 + qr / kGf, M - 1) * kGf + qr % kGf) * kDf + 8 * hf;
+#pragma unroll
+        for (int j = 0; j < 32; ++j) qf[j] = ld16(qp + 16 * j);
+    }
+    // valid slots: wave w reads row m0 + w, 16 slots per lane, 16 tiles per pass
+    {
+        const int m = m0 + wave;
+        const float* mr = mask + (size_t)min(m, M - 1) * kTf + (lane & 3) * 16;
+        for (int base = 0; base < nt; base += 16) {
+            const int u = base + (lane >> 2), a = u0 + min(u, nt - 1);
+            const float* mp = mr + (size_t)(a / kFaChunks) * mask_page_stride + a % kFaChunks * kFaChunk;
+            fa_f32x4u v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const fa_f32x4u*>(mp + 4 * i);
+            uint32_t b = 0;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) b |= v[i >> 2][i & 3] != 0.0f ? 1u << i : 0u;
+            if (u < nt) reinterpret_cast<uint16_t*>(&bits[wave][u])[lane & 3] = m < M ? (uint16_t)b : 0;
+        }
+    }
+    __syncthreads();
+    // the tiles some row has a valid slot in, in order
+    uint64_t todo = 0;
+    {
+        uint64_t any = 0;
+        if (lane < nt)
+#pragma unroll
+            for (int r = 0; r < kFrRows; ++r) any |= bits[r][lane];
+        todo = __ballot(any != 0);
+    }
+
+    // LDS addresses (bytes) of K chunk hf of row 32 sh + l32 (chunk 2 j + hf: 32 j flips its bits, j / 8 as 256
+    // bytes each), and of V's first read: slots 8 hf + (lane % 16) / 4 (16 kk + 4 y more: rows, and y flips
+    // the swizzle's low bit, 16 bytes), dims 128 w + 16 (lane / 16 % 2) + 4 (lane % 4) (dim tile dt: 64 dt flips)
+    const int krow = 32 * sh + l32, i16 = lane & 15, vrow = 8 * hf + (i16 >> 2);
+    const int ka = krow * 1024 + (hf ^ fr_swizzle(krow)) * 16;
+    const int va = vrow * 1024 + ((16 * wave + 2 * (lane >> 4 & 1) + (i16 >> 1 & 1)) ^ fr_swizzle(vrow)) * 16 + (i16 & 1) * 8;
+
+    f32x16 o[4][2];
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int qt = 0; qt < 2; ++qt)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) o[dt][qt][e] = 0.0f;
+    // of query row 32 qh + l32: the largest score, the score that weights are relative to, and the sum over
+    // this wave's slot half
+    float m_run = -INFINITY, m_ref = -INFINITY, l_run = 0.0f;
+
+    int u = todo ? __builtin_ctzll(todo) : 0;
+    if (u || !todo) {  // not the first tile, or none: its load ends before the rows are loaded again or the wave does
+        __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (todo) issue(krs, ks, u, 0, 16);
+    }
+    while (todo) {
+        todo &= todo - 1;
+        const int un = todo ? __builtin_ctzll(todo) : 0;
+        __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's K rows are in LDS
+        fr_barrier();                                          // and the others'; V's reads of the tile before are done
+        // four sums of 8 MFMAs, added in pairs: one long chain's rounding would show in running_sum
+        f32x16 sc[4];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sc[0][e] = sc[1][e] = sc[2][e] = sc[3][e] = 0.0f;
+        // eight K fragments ahead of the MFMAs that use them; this tile's V beside them
+        bf16x8 kf[8];
+        int kb = ka, vb0 = va;
+        __asm__ volatile("" : "+v"(kb), "+v"(vb0));  // addresses made anew per tile, as in issue
+        auto read_k = [&](int j) {
+            kf[j & 7] = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const uint8_t*>(ks) + (kb ^ (32 * (j & 7))) + (j >> 3) * 256);
+        };
+#pragma unroll
+        for (int j = 0; j < 8; ++j) read_k(j);
+#pragma unroll
+        for (int j = 0; j < 32; j += 2) {
+#pragma unroll
+            for (int i = j; i < j + 2; ++i)
+                sc[i & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i & 7], as_bf16x8(qf[i]), sc[i & 3], 0, 0, 0);
+            if (j < 24) {
+                read_k(j + 8);
+                read_k(j + 9);
+            }
+            issue(vrs, vs, u, j / 2, j / 2 + 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // element e: slot 32 sh + 8 (e / 4) + 4 hf + e % 4
+        const uint32_t vb = (uint32_t)(bits[2 * qh + (l32 >> 4)][u] >> (32 * sh + 4 * hf));
+        float mx = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sc[0][e] = (sc[0][e] + sc[1][e]) + (sc[2][e] + sc[3][e]);
+        if (!__all((vb & 0x0f0f0f0fu) == 0x0f0f0f0fu)) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) sc[0][e] = (vb >> (8 * (e >> 2) + (e & 3)) & 1) ? sc[0][e] : -INFINITY;
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sc[0][e]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        if (hf == 0) red[sh][32 * qh + l32] = mx;
+        fr_barrier();  // maxima; K's reads are done
+        m_run = fmaxf(m_run, fmaxf(red[0][32 * qh + l32], red[1][32 * qh + l32]));
+        float scale = 1.0f;
+        if (m_run > m_ref + kFrSlack) {
+            scale = m_ref == -INFINITY ? 1.0f : __expf(m_ref - m_run);  // -inf: sum and out are still zero
+            m_ref = m_run;
+        }
+        const float mu = m_ref == -INFINITY ? 0.0f : m_ref;
+        float ls = 0.0f;
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            if (todo) issue(krs, ks, un, 4 * a, 4 * a + 4);
+            float p[4], lo[4];
+            uint32_t hi[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                p[e] = __expf(sc[0][4 * a + e] - mu);
+                ls += p[e];
+                hi[e] = f2bf(p[e]);
+                lo[e] = p[e] - bf2f(hi[e]);
+            }
+            const int at = (32 * qh + l32) * kFrPStride + 32 * sh + 8 * a + 4 * hf;
+            *reinterpret_cast<uint2*>(&ps[0][at]) = make_uint2(hi[0] | hi[1] << 16, hi[2] | hi[3] << 16);
+            *reinterpret_cast<uint2*>(&ps[1][at]) = make_uint2(pk_bf16(lo[0], lo[1]), pk_bf16(lo[2], lo[3]));
+        }
+        l_run = fmaf(l_run, scale, ls + __shfl_xor(ls, 32));
+        if (sh == 0 && hf == 0) scl[32 * qh + l32] = scale;
+        // V's rows are in LDS (behind them only the next K tile's 16 loads); weights and scales too
+        if (todo) __asm__ volatile("s_waitcnt vmcnt(16)" ::: "memory");
+        else __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        fr_barrier();
+#pragma unroll
+        for (int qt = 0; qt < 2; ++qt) {
+            const float f = scl[32 * qt + l32];
+            if (__any(f != 1.0f)) {
+#pragma unroll
+                for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) o[dt][qt][e] *= f;
+            }
+        }
+        // step n: slots 16 (n / 4) .. + 15, dim tile n % 4; V two steps ahead, the weights three
+        bf16x8 pb[2][2][2], vf[3];
+        auto read_p = [&](bf16x8 (&d)[2][2], int kk) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int qt = 0; qt < 2; ++qt)
+                    d[h][qt] = *reinterpret_cast<const bf16x8*>(&ps[h][(32 * qt + l32) * kFrPStride + 16 * kk + 8 * hf]);
+        };
+        auto read_v = [&](bf16x8& d, int n) {
+            fa_s16x4 a[2];
+#pragma unroll
+            for (int y = 0; y < 2; ++y)
+                a[y] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (fa_lds_s16x4*)(reinterpret_cast<uint8_t*>(vs) + (vb0 ^ (64 * (n & 3) + 16 * y)) + ((n >> 2) * 16 + 4 * y) * 1024));
+            d = __builtin_bit_cast(bf16x8, __builtin_shufflevector(a[0], a[1], 0, 1, 2, 3, 4, 5, 6, 7));
+        };
+        read_p(pb[0], 0);
+        read_v(vf[0], 0);
+        read_v(vf[1], 1);
+#pragma unroll
+        for (int n = 0; n < 16; ++n) {
+            if (n < 14) read_v(vf[(n + 2) % 3], n + 2);
+            if (n % 4 == 1 && n < 12) read_p(pb[(n / 4 + 1) & 1], n / 4 + 1);
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int qt = 0; qt < 2; ++qt)
+                    o[n & 3][qt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[n % 3], pb[n / 4 & 1][h][qt], o[n & 3][qt], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        u = un;
+    }
+    // the sums of the slot halves, and the factor that brings the state to the maximum
+    fr_barrier();
+    const float fin = m_ref == -INFINITY ? 0.0f : __expf(m_ref - m_run);
+    if (hf == 0) {
+        red[sh][32 * qh + l32] = l_run;
+        if (sh == 0) scl[32 * qh + l32] = fin;
+    }
+    fr_barrier();
+    if (sh == 0 && hf == 0) {
+        const int qr = 32 * qh + l32, m = m0 + qr / kGf;
+        if (m < M) {
+            float* pc = part + ((size_t)m * gridDim.x + blockIdx.x) * kFaRec;
+            pc[qr % kGf] = m_run;
+            pc[kGf + qr % kGf] = (red[0][qr] + red[1][qr]) * fin;
+        }
+    }
+    // out through LDS (over K and V: 32 query rows of 2 KB each, 16-byte chunks permuted so that neither
+    // side meets on banks), so that a wave stores whole 1 KB runs of a record
+#pragma unroll
+    for (int qt = 0; qt < 2; ++qt) {
+        uint8_t* os = reinterpret_cast<uint8_t*>(qt ? vs : ks);
+        const float f = scl[32 * qt + l32];
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+                *reinterpret_cast<float4*>(os + l32 * 2048 + ((32 * wave + 8 * dt + 2 * a + hf) ^ (l32 & 15)) * 16) =
+                    make_float4(o[dt][qt][4 * a] * f, o[dt][qt][4 * a + 1] * f, o[dt][qt][4 * a + 2] * f,
+                                o[dt][qt][4 * a + 3] * f);
+    }
+    fr_barrier();
+#pragma unroll
+    for (int i = 0; i < kFrQ / 4; ++i) {
+        const int qr = 4 * i + wave, m = m0 + qr / kGf;
+        if (m >= M) continue;
+        const uint8_t* os = reinterpret_cast<const uint8_t*>(qr >= 32 ? vs : ks) + (qr & 31) * 2048;
+        float* pc = part + ((size_t)m * gridDim.x + blockIdx.x) * kFaRec + 2 * kGf + qr % kGf * kDf;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            *reinterpret_cast<float4*>(pc + 4 * (64 * h + lane)) =
+                *reinterpret_cast<const float4*>(os + ((64 * h + lane) ^ (qr & 15)) * 16);
+    }
+}
+
+// Workgroup (h, m) merges head h's nrec (at most 8) records into the row's state; thread t owns dims
 // 2 t, 2 t + 1.
-__global__ __launch_bounds__(kFaBlock) void fattn_combine_kernel(const float* __restrict__ part, float* rmax,
+__global__ __launch_bounds__(kFaBlock) void fattn_combine_kernel(const float* __restrict__ part, int nrec, float* rmax,
                                                                  float* rsum, uint16_t* out, int first) {
     const int h = blockIdx.x, m = blockIdx.y, t = threadIdx.x;
-    const float* pm = part + (size_t)m * kFaChunks * kFaRec;
+    const float* pm = part + (size_t)m * nrec * kFaRec;
     float mc[kFaChunks], lc[kFaChunks];
     float2 oc[kFaChunks];
 #pragma unroll
     for (int c = 0; c < kFaChunks; ++c) {
-        mc[c] = pm[c * kFaRec + h];
-        lc[c] = pm[c * kFaRec + kGf + h];
-        oc[c] = *reinterpret_cast<const float2*>(pm + c * kFaRec + 2 * kGf + h * kDf + 2 * t);
+        const float* rec = pm + min(c, nrec - 1) * kFaRec;
+        mc[c] = c < nrec ? rec[h] : -INFINITY;
+        lc[c] = rec[kGf + h];
+        oc[c] = *reinterpret_cast<const float2*>(rec + 2 * kGf + h * kDf + 2 * t);
     }
     const size_t sh = (size_t)m * kGf + h;
     uint32_t* op = reinterpret_cast<uint32_t*>(out + sh * kDf) + t;
@@ -417,8 +709,9 @@ __global__ __launch_bounds__(kFaBlock) void fattn_combine_kernel(const float* __
 // LDS in a fixed order. Records of chunks with no valid slot hold max -inf and add nothing.
 constexpr int kFmGroups = 8;
 constexpr int kFmDims = 64;
-constexpr int kFmRpg = kFaMaxRecords / kFmGroups;
 
+// RPG: the most records per group (every load of them is issued, those past nrec again for the last).
+template <int RPG>
 __global__ __launch_bounds__(kFaBlock) void fattn_merge_kernel(const float* __restrict__ part, int nrec, float* rmax,
                                                                float* rsum, uint16_t* out) {
     __shared__ float wm[kFmGroups], wl[kFmGroups];
@@ -427,10 +720,10 @@ __global__ __launch_bounds__(kFaBlock) void fattn_merge_kernel(const float* __re
     const int t = threadIdx.x, rg = t / (kFmDims / 2), dp = t % (kFmDims / 2);
     const float* pm = part + (size_t)m * nrec * kFaRec;
     const int d = db * kFmDims + 2 * dp;
-    float mr[kFmRpg], lr[kFmRpg];
-    float2 ov[kFmRpg];
+    float mr[RPG], lr[RPG];
+    float2 ov[RPG];
 #pragma unroll
-    for (int i = 0; i < kFmRpg; ++i) {
+    for (int i = 0; i < RPG; ++i) {
         const int x = rg + kFmGroups * i;
         const float* rec = pm + (size_t)min(x, nrec - 1) * kFaRec;
         mr[i] = x < nrec ? rec[h] : -INFINITY;
@@ -439,7 +732,7 @@ __global__ __launch_bounds__(kFaBlock) void fattn_merge_kernel(const float* __re
     }
     float mw = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < kFmRpg; ++i) mw = fmaxf(mw, mr[i]);
+    for (int i = 0; i < RPG; ++i) mw = fmaxf(mw, mr[i]);
     if (dp == 0) wm[rg] = mw;
     __syncthreads();
     float mx = -INFINITY;
@@ -448,7 +741,7 @@ __global__ __launch_bounds__(kFaBlock) void fattn_merge_kernel(const float* __re
     float l = 0.0f, o0 = 0.0f, o1 = 0.0f;
     if (mx != -INFINITY) {
 #pragma unroll
-        for (int i = 0; i < kFmRpg; ++i) {
+        for (int i = 0; i < RPG; ++i) {
             const float f = mr[i] == -INFINITY ? 0.0f : __expf(mr[i] - mx);
             l = fmaf(f, lr[i], l);
             o0 = fmaf(f, ov[i].x, o0);
@@ -476,31 +769,66 @@ __global__ __launch_bounds__(kFaBlock) void fattn_merge_kernel(const float* __re
 
 }  // namespace
 
+// Rows m0 .. m0 + mm - 1 of the merge; P pages in nrec records per row.
+static hipError_t merge_rows(const float* part, int nrec, float* rmax, float* rsum, uint16_t* out, int mm, hipStream_t s) {
+    const dim3 grid(kGf, kDf / kFmDims, mm), block(kFaBlock);
+    if (nrec <= kFaChunks)  // few records: a workgroup per head
+        hipLaunchKernelGGL(fattn_combine_kernel, dim3(kGf, mm), block, 0, s, part, nrec, rmax, rsum, out, 1);
+    else if (nrec <= 4 * kFmGroups) hipLaunchKernelGGL(fattn_merge_kernel<4>, grid, block, 0, s, part, nrec, rmax, rsum, out);
+    else if (nrec <= 8 * kFmGroups) hipLaunchKernelGGL(fattn_merge_kernel<8>, grid, block, 0, s, part, nrec, rmax, rsum, out);
+    else hipLaunchKernelGGL(fattn_merge_kernel<kFaMaxRecords / kFmGroups>, grid, block, 0, s, part, nrec, rmax, rsum, out);
+    return hipGetLastError();
+}
+
+// The split of fattn_rows_kernel for M rows over ntiles tiles: records per row, tiles per record and rows
+// per launch. About one workgroup per CU (one fits a CU), at most kFrMaxTiles tiles each, and the
+// records of a launch within the scratch.
+struct RowsSplit {
+    int nrec, tpw, rows;
+};
+static RowsSplit rows_split(int M, int ntiles, int cus) {
+    const int blocks = ((M < kFattnRecords ? M : kFattnRecords) + kFrRows - 1) / kFrRows;
+    int n = cus / blocks;
+    n = n < 1 ? 1 : (n > kFaMaxRecords ? kFaMaxRecords : n);
+    if (n > ntiles) n = ntiles;
+    if (n * kFrMaxTiles < ntiles) n = (ntiles + kFrMaxTiles - 1) / kFrMaxTiles;
+    RowsSplit r;
+    r.tpw = (ntiles + n - 1) / n;
+    r.nrec = (ntiles + r.tpw - 1) / r.tpw;
+    r.rows = kFattnRecords / r.nrec;  // at least kFrRows: nrec <= kFaMaxRecords
+    return r;
+}
+static_assert(kFattnRecords >= kFrRows * kFaMaxRecords, "a launch of fattn_rows_kernel holds four rows");
+
 hipError_t launch_full_attention(const uint16_t* q, const uint16_t* k_pages, const uint16_t* v_pages,
                                  const float* masks, int P, float* running_max, float* running_sum, uint16_t* out,
                                  int M, hipStream_t s, DevCtx* ctx) {
     const int nchunks = P * kFaChunks;
-    // Up to kFaSplitPages pages: one chunk per dim-split workgroup (P x 32 workgroups). More: spans
-    // of chunks over all dims, at most kFaMaxRecords workgroups per row.
+    const bool many = M * P >= kFrMinRowPages;
+    // One row, up to kFaSplitPages pages: one chunk per dim-split workgroup (P x 32 workgroups). More:
+    // spans of chunks over all dims, at most kFaMaxRecords workgroups per row.
     const bool split = P <= kFaSplitPages;
-    const int cpw = split ? 1 : (nchunks + kFaMaxRecords - 1) / kFaMaxRecords;
-    const int nrec = (nchunks + cpw - 1) / cpw;
-    const int rows = kFattnRecords / nrec;  // rows per launch (scratch)
-    for (int m0 = 0; m0 < M; m0 += rows) {
-        const int mm = M - m0 < rows ? M - m0 : rows;
-        if (split)
-            hipLaunchKernelGGL(fattn_partial_kernel, dim3(nrec, kFaDimBlocks, mm), dim3(kFaBlock), 0, s,
-                               q + (size_t)m0 * kQf, k_pages, v_pages, masks + (size_t)m0 * kTf, M * kTf, nchunks,
-                               cpw, ctx->fattn_part);
+    RowsSplit r = {0, split ? 1 : (nchunks + kFaMaxRecords - 1) / kFaMaxRecords, 1};
+    r.nrec = (nchunks + r.tpw - 1) / r.tpw;
+    if (many) r = rows_split(M, nchunks, ctx->cus);
+    else r.rows = kFattnRecords / r.nrec;
+    for (int m0 = 0; m0 < M; m0 += r.rows) {
+        const int mm = M - m0 < r.rows ? M - m0 : r.rows;
+        const uint16_t* qm = q + (size_t)m0 * kQf;
+        const float* mk = masks + (size_t)m0 * kTf;
+        if (many)
+            hipLaunchKernelGGL(fattn_rows_kernel, dim3(r.nrec, (mm + kFrRows - 1) / kFrRows), dim3(kFaBlock), 0, s, qm,
+                               k_pages, v_pages, mk, M * kTf, mm, nchunks, r.tpw, ctx->fattn_part);
+        else if (split)
+            hipLaunchKernelGGL(fattn_partial_kernel, dim3(r.nrec, kFaDimBlocks, mm), dim3(kFaBlock), 0, s, qm, k_pages,
+                               v_pages, mk, M * kTf, nchunks, r.tpw, ctx->fattn_part);
         else
-            hipLaunchKernelGGL(fattn_span_kernel, dim3(nrec, 1, mm), dim3(kFaBlock), 0, s, q + (size_t)m0 * kQf,
-                               k_pages, v_pages, masks + (size_t)m0 * kTf, M * kTf, nchunks, cpw, ctx->fattn_part);
+            hipLaunchKernelGGL(fattn_span_kernel, dim3(r.nrec, 1, mm), dim3(kFaBlock), 0, s, qm, k_pages, v_pages, mk,
+                               M * kTf, nchunks, r.tpw, ctx->fattn_part);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(fattn_merge_kernel, dim3(kGf, kDf / kFmDims, mm), dim3(kFaBlock), 0, s,
-                           (const float*)ctx->fattn_part, nrec, running_max + (size_t)m0 * kGf,
-                           running_sum + (size_t)m0 * kGf, out + (size_t)m0 * kQf);
-        e = hipGetLastError();
+        e = merge_rows(ctx->fattn_part, r.nrec, running_max + (size_t)m0 * kGf, running_sum + (size_t)m0 * kGf,
+                       out + (size_t)m0 * kQf, mm, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -509,14 +837,22 @@ hipError_t launch_full_attention(const uint16_t* q, const uint16_t* k_pages, con
 hipError_t launch_full_attention_page(const uint16_t* q, const uint16_t* k_page, const uint16_t* v_page,
                                       const float* mask, float* running_max, float* running_sum, uint16_t* out,
                                       int M, bool first, hipStream_t s, DevCtx* ctx) {
-    for (int m0 = 0; m0 < M; m0 += kMaxDecodeM) {
-        const int mm = M - m0 < kMaxDecodeM ? M - m0 : kMaxDecodeM;
-        hipLaunchKernelGGL(fattn_partial_kernel, dim3(kFaChunks, kFaDimBlocks, mm), dim3(kFaBlock), 0, s,
-                           q + (size_t)m0 * kQf, k_page, v_page, mask + (size_t)m0 * kTf, 0, kFaChunks, 1,
-                           ctx->fattn_part);
+    // Many rows share a pass over the page (kFaChunks tiles, at most as many records per row)
+    const bool many = M >= kFrMinPageRows;
+    const RowsSplit r = many ? rows_split(M, kFaChunks, ctx->cus) : RowsSplit{kFaChunks, 1, kMaxDecodeM};
+    for (int m0 = 0; m0 < M; m0 += r.rows) {
+        const int mm = M - m0 < r.rows ? M - m0 : r.rows;
+        if (many)
+            hipLaunchKernelGGL(fattn_rows_kernel, dim3(r.nrec, (mm + kFrRows - 1) / kFrRows), dim3(kFaBlock), 0, s,
+                               q + (size_t)m0 * kQf, k_page, v_page, mask + (size_t)m0 * kTf, 0, mm, kFaChunks, r.tpw,
+                               ctx->fattn_part);
+        else
+            hipLaunchKernelGGL(fattn_partial_kernel, dim3(kFaChunks, kFaDimBlocks, mm), dim3(kFaBlock), 0, s,
+                               q + (size_t)m0 * kQf, k_page, v_page, mask + (size_t)m0 * kTf, 0, kFaChunks, 1,
+                               ctx->fattn_part);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(fattn_combine_kernel, dim3(kGf, mm), dim3(kFaBlock), 0, s, (const float*)ctx->fattn_part,
+        hipLaunchKernelGGL(fattn_combine_kernel, dim3(kGf, mm), dim3(kFaBlock), 0, s, (const float*)ctx->fattn_part, r.nrec,
                            running_max + (size_t)m0 * kGf, running_sum + (size_t)m0 * kGf, out + (size_t)m0 * kQf,
                            first ? 1 : 0);
         e = hipGetLastError();
