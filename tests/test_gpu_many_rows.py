@@ -43,13 +43,13 @@ def test_sliding_attention_rows(M, kind):
         d["mask"] = (rng.random((M, TS)) < 0.3).astype(np.float32) * np.float32(-2.5)  # any non-zero value counts
     if kind == "empty":
         d["mask"][:, 64:700] = 0.0
-        d["mask"][5] = 0.0
+        d["mask"][3] = 0.0
         d["mask"][M - 1] = 0.0
         d["mask"][M - 1, 1023] = 1.0
     got = run_gpu(d)
     gate(run_oracle(d), got, f"attention M{M} {kind}")
     if kind == "empty":
-        assert not got[5].any()
+        assert not got[3].any()
         v = d["v_cache"].reshape(TS, 8, 256)[1023]
         assert np.array_equal(got[M - 1], np.repeat(v[:, None, :], 2, axis=1))
 
