@@ -368,28 +368,33 @@ __global__ __launch_bounds__(kFaBlock) void fattn_span_kernel(const uint16_t* __
 // Several token rows: all their heads share the one KV head, so a tile of 64 slots is read once for
 // four rows (64 query rows of 512). Workgroup (x, y): rows 4 y .. 4 y + 3, tiles x * tpw .. (64
 // slots; a page holds 8), an online softmax over those of its tiles in which some row has a valid
-// slot; record x of each row. On v_mfma_f32_32x32x16_bf16, transposed, so that a lane holds one
-// query row's values:
-//   scores^T = K Q^T: wave (sh, qh) takes 32 of the slots and 32 of the query rows, whose 512 dims stay in
-//     registers; the two slot halves exchange their maxima through LDS, sums stay apart to the end;
-//   out^T += V^T P^T: wave w takes dims 128 w .. + 127 of all 64 query rows, over the weights of both
-//     slot halves from LDS (bf16 high and low parts, as in the kernels above).
+// slot; record x of each row. Eight waves, two per SIMD, on the matrix cores, transposed, so that a lane
+// holds one query row's values:
+//   scores^T = K Q^T (16x16x32): wave (sh, r) takes 32 of the slots and the 16 heads of row r, whose 512 dims
+//     stay in registers; the slot halves exchange their maxima through LDS, sums stay apart to the end;
+//   out^T += V^T P^T (32x32x16): wave w takes dims 64 w .. + 63 of all 64 query rows, over the weights of
+//     both slot halves from LDS (bf16 high and low parts, as in the kernels above).
 // K and V tiles go straight to LDS (16-byte chunks of a row permuted by fr_swizzle, so that neither
-// the K rows' reads nor V's transposing reads meet on banks): the next tile's K while the
-// weights and out are computed, its V while its scores are. 96 MFMAs a tile and wave.
+// the K rows' reads nor V's transposing reads meet on banks): the next tile's K beside out's
+// products, this tile's V beside its scores. Bound by LDS: 450 KB of fragments a tile, 3500 cycles, beside 3100 of
+// MFMAs. 200 rows over 6 pages (18 GFLOP, 34 MB of records): 48 us, and 7-10 for the merge; 4 rows over 64 pages
+// (67 MB of K and V): 21-23 and 7. (Four waves of 512 registers instead kept Q and out in accumulation registers and
+// copied them around the MFMAs: 60 us.)
+constexpr int kFrBlock = 512;
 constexpr int kFrRows = 4;                      // token rows per workgroup
 constexpr int kFrQ = kFrRows * kGf;             // query rows
 constexpr int kFrMaxTiles = 64;                 // tiles per workgroup
 constexpr int kFrPStride = kFaChunk + 8;        // LDS row of the weights, in elements
 // Weights are exp(score - reference) with a reference at most this far below the row's largest score: out
-// (128 accumulators a lane) is rescaled only when the maximum has grown by more, which after the
-// first tile it hardly does, not at every new maximum. The state is brought to the maximum at the end.
+// (64 accumulators a lane) is rescaled only when the maximum has grown by more. The state is brought to
+// the maximum at the end.
 constexpr float kFrSlack = 8.0f;
 // From these row x pages products of a call over all pages (rows of a one-page call) on this path is used.
-// All pages, this path against the one-row kernels on every row: M x P = 2 x 8 18.2 / 15.8 us, 4 x 3 19.0 /
-// 15.2, 16 x 1 19.8 / 16.2, 3 x 8 21.0 / 21.4, 13 x 3 23.7 / 34.0, 2 x 64 29.1 / 37.3, 200 x 6 66 / 840.
-// One page: 16 rows 18.4 / 15.1 us; more would be several launches of the one-row kernel (64 rows 25.6 / 59.2).
-constexpr int kFrMinRowPages = 24;
+// All pages, this path against the one-row kernels on every row: M x P = 2 x 4 13.5 / 9.9 us, 4 x 3 15.4 /
+// 15.4, 2 x 8 15.1 / 15.8, 16 x 1 15.9 / 16.5, 2 x 12 17.2 / 15.6, 3 x 8 17.1 / 21.7, 13 x 3 19.2 / 34.0, 2 x 64
+// 25.1 / 37.0, 200 x 6 54 / 839. One page: up to 16 rows one launch of the one-row kernel (15 us); more would be
+// several (64 rows 22.0 / 59.2, 200 rows 27 / 191).
+constexpr int kFrMinRowPages = 16;
 constexpr int kFrMinPageRows = 17;
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef short fa_s16x4 __attribute__((ext_vector_type(4)));
@@ -407,7 +412,7 @@ __device__ __forceinline__ void fr_barrier() {
     __asm__ volatile("" ::: "memory");
 }
 
-__global__ __launch_bounds__(kFaBlock) __attribute__((amdgpu_waves_per_eu(1, 1))) void fattn_rows_kernel(
+__global__ __launch_bounds__(kFrBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) void fattn_rows_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     const float* __restrict__ mask, int mask_page_stride, int M, int ntiles, int tpw, float* part) {
     __shared__ __attribute__((aligned(1024))) uint16_t ks[kFaChunk * kDf];
@@ -416,40 +421,37 @@ __global__ __launch_bounds__(kFaBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
     __shared__ uint64_t bits[kFrRows][kFrMaxTiles];   // bit s: slot s of the tile is valid for the row
     __shared__ float red[2][kFrQ], scl[kFrQ];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int l32 = lane & 31, hf = lane >> 5;
+    const int l32 = lane & 31, hf = lane >> 5, l16 = lane & 15, g = lane >> 4;
     const int m0 = blockIdx.y * kFrRows;
     const int u0 = blockIdx.x * tpw, nt = min(tpw, ntiles - u0);
-    const int sh = wave & 1, qh = wave >> 1;
+    const int sh = wave & 1, row = wave >> 1, qr = kGf * row + l16;  // the wave's part of the scores; the lane's query row
 
-    // K or V tile u into LDS: wave w moves rows 16 w .. 16 w + 15, a row (1 KB) per instruction
+    // K or V tile u into LDS: wave w moves rows 8 w .. 8 w + 7 (of those, i0 .. i1 - 1), a row (1 KB) per instruction
     const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(kc + (size_t)u0 * kFaChunk * kDf), 0, (uint32_t)nt * kFaChunk * kDf * 2, 0x00020000);
     const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(vc + (size_t)u0 * kFaChunk * kDf), 0, (uint32_t)nt * kFaChunk * kDf * 2, 0x00020000);
-    // (rows i0 .. i1 - 1 of the wave's 16; the loads are spread over other work: issued together they hold the
-    // wave for a thousand cycles)
     auto issue = [&](__amdgpu_buffer_rsrc_t rs, uint16_t* dst, int u, int i0, int i1) {
-        int ln = lane;
-        __asm__ volatile("" : "+v"(ln));  // the 16 permuted offsets are made anew: kept, they would not fit the registers
 #pragma unroll
-        for (int i = i0; i < i1; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (fa_lds_void*)(dst + (wave * 16 + i) * kDf), 16,
-                                                     (ln ^ fr_swizzle(i)) * 16, (u * kFaChunk + wave * 16 + i) * kDf * 2, 0, 0);
+        for (int i = i0; i < i1; ++i) {
+            const int r = wave * 8 + i;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (fa_lds_void*)(dst + r * kDf), 16, (lane ^ fr_swizzle(r)) * 16,
+                                                     (u * kFaChunk + r) * kDf * 2, 0, 0);
+        }
     };
-    issue(krs, ks, 0, 0, 16);  // most often the first tile it needs (else read again)
-    // Q: lane (l32, hf) holds query row 32 qh + l32, dims 16 j + 8 hf .. + 7 (a row past M repeats the last)
-    uint4 qf[32];
+    issue(krs, ks, 0, 0, 8);  // most often the first tile it needs (else read again)
+    // Q: lane (l16, g) holds dims 32 j + 8 g .. + 7 of its query row (a row past M repeats the last)
+    uint4 qf[16];
     {
-        const int qr = 32 * qh + l32;
-        const uint16_t* qp = q + ((size_t)min(m0 + qr / kGf, M - 1) * kGf + qr % kGf) * kDf + 8 * hf;
+        const uint16_t* qp = q + ((size_t)min(m0 + row, M - 1) * kGf + l16) * kDf + 8 * g;
 #pragma unroll
-        for (int j = 0; j < 32; ++j) qf[j] = ld16(qp + 16 * j);
+        for (int j = 0; j < 16; ++j) qf[j] = ld16(qp + 32 * j);
     }
-    // valid slots: wave w reads row m0 + w, 16 slots per lane, 16 tiles per pass
+    // valid slots: waves r and r + 4 read row m0 + r, 16 slots per lane, 16 tiles per pass
     {
-        const int m = m0 + wave;
+        const int r = wave & 3, m = m0 + r;
         const float* mr = mask + (size_t)min(m, M - 1) * kTf + (lane & 3) * 16;
-        for (int base = 0; base < nt; base += 16) {
+        for (int base = 16 * (wave >> 2); base < nt; base += 32) {
             const int u = base + (lane >> 2), a = u0 + min(u, nt - 1);
             const float* mp = mr + (size_t)(a / kFaChunks) * mask_page_stride + a % kFaChunks * kFaChunk;
             fa_f32x4u v[4];
@@ -458,7 +460,7 @@ __global__ __launch_bounds__(kFaBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
             uint32_t b = 0;
 #pragma unroll
             for (int i = 0; i < 16; ++i) b |= v[i >> 2][i & 3] != 0.0f ? 1u << i : 0u;
-            if (u < nt) reinterpret_cast<uint16_t*>(&bits[wave][u])[lane & 3] = m < M ? (uint16_t)b : 0;
+            if (u < nt) reinterpret_cast<uint16_t*>(&bits[r][u])[lane & 3] = m < M ? (uint16_t)b : 0;
         }
     }
     __syncthreads();
@@ -472,74 +474,75 @@ __global__ __launch_bounds__(kFaBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
         todo = __ballot(any != 0);
     }
 
-    // LDS addresses (bytes) of K chunk hf of row 32 sh + l32 (chunk 2 j + hf: 32 j flips its bits, j / 8 as 256
-    // bytes each), and of V's first read: slots 8 hf + (lane % 16) / 4 (16 kk + 4 y more: rows, and y flips
-    // the swizzle's low bit, 16 bytes), dims 128 w + 16 (lane / 16 % 2) + 4 (lane % 4) (dim tile dt: 64 dt flips)
-    const int krow = 32 * sh + l32, i16 = lane & 15, vrow = 8 * hf + (i16 >> 2);
-    const int ka = krow * 1024 + (hf ^ fr_swizzle(krow)) * 16;
-    const int va = vrow * 1024 + ((16 * wave + 2 * (lane >> 4 & 1) + (i16 >> 1 & 1)) ^ fr_swizzle(vrow)) * 16 + (i16 & 1) * 8;
+    // LDS addresses (bytes). K chunk g of slot 32 sh + l16 (chunk 4 j + g: 64 j flips its bits, j / 4 as 256 bytes
+    // each; the second 16 slots as rows). V's first read: slots 8 hf + l16 / 4 (16 kk + 4 y more: rows, and y
+    // flips the swizzle's low bit, 16 bytes), dims 64 w + 16 (g % 2) + 4 (l16 % 4) (dim tile dt: 64 dt flips).
+    const int krow = 32 * sh + l16, vrow = 8 * hf + (l16 >> 2);
+    const int ka = krow * 1024 + (g ^ fr_swizzle(krow)) * 16;
+    const int va = vrow * 1024 + ((8 * wave + 2 * (g & 1) + (l16 >> 1 & 1)) ^ fr_swizzle(vrow)) * 16 + (l16 & 1) * 8;
 
-    f32x16 o[4][2];
+    f32x16 o[2][2];
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+    for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
         for (int qt = 0; qt < 2; ++qt)
 #pragma unroll
             for (int e = 0; e < 16; ++e) o[dt][qt][e] = 0.0f;
-    // of query row 32 qh + l32: the largest score, the score that weights are relative to, and the sum over
-    // this wave's slot half
+    // of the lane's query row: the largest score, the score that weights are relative to, and the sum of the
+    // weights the lane has computed
     float m_run = -INFINITY, m_ref = -INFINITY, l_run = 0.0f;
 
     int u = todo ? __builtin_ctzll(todo) : 0;
     if (u || !todo) {  // not the first tile, or none: its load ends before the rows are loaded again or the wave does
         __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        if (todo) issue(krs, ks, u, 0, 16);
+        if (todo) issue(krs, ks, u, 0, 8);
     }
     while (todo) {
         todo &= todo - 1;
         const int un = todo ? __builtin_ctzll(todo) : 0;
         __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's K rows are in LDS
         fr_barrier();                                          // and the others'; V's reads of the tile before are done
-        // four sums of 8 MFMAs, added in pairs: one long chain's rounding would show in running_sum
-        f32x16 sc[4];
+        // per 16 slots four sums of 4 MFMAs, added in pairs: one long chain's rounding would show in running_sum;
+        // fragments four ahead of the MFMAs that use them; this tile's V beside them
+        f32x4v sc[2][4];
+        bf16x8 kf[2][4];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) sc[0][e] = sc[1][e] = sc[2][e] = sc[3][e] = 0.0f;
-        // eight K fragments ahead of the MFMAs that use them; this tile's V beside them
-        bf16x8 kf[8];
-        int kb = ka, vb0 = va;
-        __asm__ volatile("" : "+v"(kb), "+v"(vb0));  // addresses made anew per tile, as in issue
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) sc[i][c] = f32x4v{0.0f, 0.0f, 0.0f, 0.0f};
         auto read_k = [&](int j) {
-            kf[j & 7] = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const uint8_t*>(ks) + (kb ^ (32 * (j & 7))) + (j >> 3) * 256);
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                kf[i][j & 3] = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const uint8_t*>(ks) + (ka ^ (64 * (j & 3))) +
+                                                                (j >> 2) * 256 + i * 16 * 1024);
         };
 #pragma unroll
-        for (int j = 0; j < 8; ++j) read_k(j);
+        for (int j = 0; j < 4; ++j) read_k(j);
 #pragma unroll
-        for (int j = 0; j < 32; j += 2) {
+        for (int j = 0; j < 16; ++j) {
 #pragma unroll
-            for (int i = j; i < j + 2; ++i)
-                sc[i & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i & 7], as_bf16x8(qf[i]), sc[i & 3], 0, 0, 0);
-            if (j < 24) {
-                read_k(j + 8);
-                read_k(j + 9);
-            }
-            issue(vrs, vs, u, j / 2, j / 2 + 1);
+            for (int i = 0; i < 2; ++i)
+                sc[i][j & 3] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[i][j & 3], as_bf16x8(qf[j]), sc[i][j & 3], 0, 0, 0);
+            if (j < 12) read_k(j + 4);
+            if (j & 1) issue(vrs, vs, u, j >> 1, (j >> 1) + 1);
             __builtin_amdgcn_sched_barrier(0);
         }
-        // element e: slot 32 sh + 8 (e / 4) + 4 hf + e % 4
-        const uint32_t vb = (uint32_t)(bits[2 * qh + (l32 >> 4)][u] >> (32 * sh + 4 * hf));
-        float mx = -INFINITY;
+        // element (i, e): slot 32 sh + 16 i + 4 g + e
+        const uint32_t vb = (uint32_t)(bits[row][u] >> (32 * sh + 4 * g));
+        float x[2][4], mx = -INFINITY;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) sc[0][e] = (sc[0][e] + sc[1][e]) + (sc[2][e] + sc[3][e]);
-        if (!__all((vb & 0x0f0f0f0fu) == 0x0f0f0f0fu)) {
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) sc[0][e] = (vb >> (8 * (e >> 2) + (e & 3)) & 1) ? sc[0][e] : -INFINITY;
-        }
-#pragma unroll
-        for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sc[0][e]);
+            for (int e = 0; e < 4; ++e) {
+                x[i][e] = (sc[i][0][e] + sc[i][1][e]) + (sc[i][2][e] + sc[i][3][e]);
+                x[i][e] = (vb >> (16 * i + e) & 1) ? x[i][e] : -INFINITY;
+                mx = fmaxf(mx, x[i][e]);
+            }
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
         mx = fmaxf(mx, __shfl_xor(mx, 32));
-        if (hf == 0) red[sh][32 * qh + l32] = mx;
+        if (g == 0) red[sh][qr] = mx;
         fr_barrier();  // maxima; K's reads are done
-        m_run = fmaxf(m_run, fmaxf(red[0][32 * qh + l32], red[1][32 * qh + l32]));
+        m_run = fmaxf(m_run, fmaxf(red[0][qr], red[1][qr]));
         float scale = 1.0f;
         if (m_run > m_ref + kFrSlack) {
             scale = m_ref == -INFINITY ? 1.0f : __expf(m_ref - m_run);  // -inf: sum and out are still zero
@@ -548,39 +551,37 @@ __global__ __launch_bounds__(kFaBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
         const float mu = m_ref == -INFINITY ? 0.0f : m_ref;
         float ls = 0.0f;
 #pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            if (todo) issue(krs, ks, un, 4 * a, 4 * a + 4);
+        for (int i = 0; i < 2; ++i) {
             float p[4], lo[4];
             uint32_t hi[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                p[e] = __expf(sc[0][4 * a + e] - mu);
+                p[e] = __expf(x[i][e] - mu);
                 ls += p[e];
                 hi[e] = f2bf(p[e]);
                 lo[e] = p[e] - bf2f(hi[e]);
             }
-            const int at = (32 * qh + l32) * kFrPStride + 32 * sh + 8 * a + 4 * hf;
+            const int at = qr * kFrPStride + 32 * sh + 16 * i + 4 * g;
             *reinterpret_cast<uint2*>(&ps[0][at]) = make_uint2(hi[0] | hi[1] << 16, hi[2] | hi[3] << 16);
             *reinterpret_cast<uint2*>(&ps[1][at]) = make_uint2(pk_bf16(lo[0], lo[1]), pk_bf16(lo[2], lo[3]));
         }
-        l_run = fmaf(l_run, scale, ls + __shfl_xor(ls, 32));
-        if (sh == 0 && hf == 0) scl[32 * qh + l32] = scale;
-        // V's rows are in LDS (behind them only the next K tile's 16 loads); weights and scales too
-        if (todo) __asm__ volatile("s_waitcnt vmcnt(16)" ::: "memory");
-        else __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        fr_barrier();
+        l_run = fmaf(l_run, scale, ls);
+        if (sh == 0 && g == 0) scl[qr] = scale;
+        __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // V's rows are in LDS
+        fr_barrier();                                          // weights and scales too
 #pragma unroll
         for (int qt = 0; qt < 2; ++qt) {
             const float f = scl[32 * qt + l32];
             if (__any(f != 1.0f)) {
 #pragma unroll
-                for (int dt = 0; dt < 4; ++dt)
+                for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
                     for (int e = 0; e < 16; ++e) o[dt][qt][e] *= f;
             }
         }
-        // step n: slots 16 (n / 4) .. + 15, dim tile n % 4; V two steps ahead, the weights three
-        bf16x8 pb[2][2][2], vf[3];
+        // Step n: slots 16 (n / 2) .. + 15, dim tile n % 2. V's fragments are all read first: the compiler waits for
+        // every load into LDS before a transposing read, so the next tile's K goes out behind them.
+        bf16x8 pb[2][2][2], vf[8];
         auto read_p = [&](bf16x8 (&d)[2][2], int kk) {
 #pragma unroll
             for (int h = 0; h < 2; ++h)
@@ -593,40 +594,40 @@ __global__ __launch_bounds__(kFaBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
 #pragma unroll
             for (int y = 0; y < 2; ++y)
                 a[y] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                    (fa_lds_s16x4*)(reinterpret_cast<uint8_t*>(vs) + (vb0 ^ (64 * (n & 3) + 16 * y)) + ((n >> 2) * 16 + 4 * y) * 1024));
+                    (fa_lds_s16x4*)(reinterpret_cast<uint8_t*>(vs) + (va ^ (64 * (n & 1) + 16 * y)) + ((n >> 1) * 16 + 4 * y) * 1024));
             d = __builtin_bit_cast(bf16x8, __builtin_shufflevector(a[0], a[1], 0, 1, 2, 3, 4, 5, 6, 7));
         };
         read_p(pb[0], 0);
-        read_v(vf[0], 0);
-        read_v(vf[1], 1);
 #pragma unroll
-        for (int n = 0; n < 16; ++n) {
-            if (n < 14) read_v(vf[(n + 2) % 3], n + 2);
-            if (n % 4 == 1 && n < 12) read_p(pb[(n / 4 + 1) & 1], n / 4 + 1);
+        for (int n = 0; n < 8; ++n) read_v(vf[n], n);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = 0; n < 8; ++n) {
+            if (todo) issue(krs, ks, un, n, n + 1);
+            if (n % 2 == 0 && n < 6) read_p(pb[(n / 2 + 1) & 1], n / 2 + 1);
 #pragma unroll
             for (int h = 0; h < 2; ++h)
 #pragma unroll
                 for (int qt = 0; qt < 2; ++qt)
-                    o[n & 3][qt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[n % 3], pb[n / 4 & 1][h][qt], o[n & 3][qt], 0, 0, 0);
+                    o[n & 1][qt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[n], pb[n / 2 & 1][h][qt], o[n & 1][qt], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         }
         u = un;
     }
-    // the sums of the slot halves, and the factor that brings the state to the maximum
+    // the sums of the lane groups and slot halves, and the factor that brings the state to the maximum
     fr_barrier();
     const float fin = m_ref == -INFINITY ? 0.0f : __expf(m_ref - m_run);
-    if (hf == 0) {
-        red[sh][32 * qh + l32] = l_run;
-        if (sh == 0) scl[32 * qh + l32] = fin;
+    l_run += __shfl_xor(l_run, 16);
+    l_run += __shfl_xor(l_run, 32);
+    if (g == 0) {
+        red[sh][qr] = l_run;
+        if (sh == 0) scl[qr] = fin;
     }
     fr_barrier();
-    if (sh == 0 && hf == 0) {
-        const int qr = 32 * qh + l32, m = m0 + qr / kGf;
-        if (m < M) {
-            float* pc = part + ((size_t)m * gridDim.x + blockIdx.x) * kFaRec;
-            pc[qr % kGf] = m_run;
-            pc[kGf + qr % kGf] = (red[0][qr] + red[1][qr]) * fin;
-        }
+    if (sh == 0 && g == 0 && m0 + row < M) {
+        float* pc = part + ((size_t)(m0 + row) * gridDim.x + blockIdx.x) * kFaRec;
+        pc[l16] = m_run;
+        pc[kGf + l16] = (red[0][qr] + red[1][qr]) * fin;
     }
     // out through LDS (over K and V: 32 query rows of 2 KB each, 16-byte chunks permuted so that neither
     // side meets on banks), so that a wave stores whole 1 KB runs of a record
@@ -635,24 +636,24 @@ __global__ __launch_bounds__(kFaBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
         uint8_t* os = reinterpret_cast<uint8_t*>(qt ? vs : ks);
         const float f = scl[32 * qt + l32];
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
+        for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
             for (int a = 0; a < 4; ++a)
-                *reinterpret_cast<float4*>(os + l32 * 2048 + ((32 * wave + 8 * dt + 2 * a + hf) ^ (l32 & 15)) * 16) =
+                *reinterpret_cast<float4*>(os + l32 * 2048 + ((16 * wave + 8 * dt + 2 * a + hf) ^ (l32 & 15)) * 16) =
                     make_float4(o[dt][qt][4 * a] * f, o[dt][qt][4 * a + 1] * f, o[dt][qt][4 * a + 2] * f,
                                 o[dt][qt][4 * a + 3] * f);
     }
     fr_barrier();
 #pragma unroll
-    for (int i = 0; i < kFrQ / 4; ++i) {
-        const int qr = 4 * i + wave, m = m0 + qr / kGf;
+    for (int i = 0; i < kFrQ / 8; ++i) {
+        const int r = 8 * i + wave, m = m0 + r / kGf;
         if (m >= M) continue;
-        const uint8_t* os = reinterpret_cast<const uint8_t*>(qr >= 32 ? vs : ks) + (qr & 31) * 2048;
-        float* pc = part + ((size_t)m * gridDim.x + blockIdx.x) * kFaRec + 2 * kGf + qr % kGf * kDf;
+        const uint8_t* os = reinterpret_cast<const uint8_t*>(r >= 32 ? vs : ks) + (r & 31) * 2048;
+        float* pc = part + ((size_t)m * gridDim.x + blockIdx.x) * kFaRec + 2 * kGf + r % kGf * kDf;
 #pragma unroll
         for (int h = 0; h < 2; ++h)
             *reinterpret_cast<float4*>(pc + 4 * (64 * h + lane)) =
-                *reinterpret_cast<const float4*>(os + ((64 * h + lane) ^ (qr & 15)) * 16);
+                *reinterpret_cast<const float4*>(os + ((64 * h + lane) ^ (r & 15)) * 16);
     }
 }
 
@@ -817,7 +818,7 @@ hipError_t launch_full_attention(const uint16_t* q, const uint16_t* k_pages, con
         const uint16_t* qm = q + (size_t)m0 * kQf;
         const float* mk = masks + (size_t)m0 * kTf;
         if (many)
-            hipLaunchKernelGGL(fattn_rows_kernel, dim3(r.nrec, (mm + kFrRows - 1) / kFrRows), dim3(kFaBlock), 0, s, qm,
+            hipLaunchKernelGGL(fattn_rows_kernel, dim3(r.nrec, (mm + kFrRows - 1) / kFrRows), dim3(kFrBlock), 0, s, qm,
                                k_pages, v_pages, mk, M * kTf, mm, nchunks, r.tpw, ctx->fattn_part);
         else if (split)
             hipLaunchKernelGGL(fattn_partial_kernel, dim3(r.nrec, kFaDimBlocks, mm), dim3(kFaBlock), 0, s, qm, k_pages,
@@ -843,7 +844,7 @@ hipError_t launch_full_attention_page(const uint16_t* q, const uint16_t* k_page,
     for (int m0 = 0; m0 < M; m0 += r.rows) {
         const int mm = M - m0 < r.rows ? M - m0 : r.rows;
         if (many)
-            hipLaunchKernelGGL(fattn_rows_kernel, dim3(r.nrec, (mm + kFrRows - 1) / kFrRows), dim3(kFaBlock), 0, s,
+            hipLaunchKernelGGL(fattn_rows_kernel, dim3(r.nrec, (mm + kFrRows - 1) / kFrRows), dim3(kFrBlock), 0, s,
                                q + (size_t)m0 * kQf, k_page, v_page, mask + (size_t)m0 * kTf, 0, mm, kFaChunks, r.tpw,
                                ctx->fattn_part);
         else
