@@ -250,7 +250,7 @@ int moa_full_attention_page(const uint16_t* q, const uint16_t* k, const uint16_t
                             float* running_max, float* running_sum, uint16_t* out, int M, void* stream);
 
 /* The state that full_attention_first_page followed by full_attention_page over pages 1 .. P-1
- * leaves, in two launches whatever P is (no counterpart in the reference, whose runtime launches
+ * leaves, in one pass over all pages (no counterpart in the reference, whose runtime launches
  * one operator per page, FO/src/host/runtime.rs:496-517). k_pages, v_pages bf16 [P,512,512]
  * contiguous (page p at p * 512 * 512); masks f32 [P,M,512]; 1 <= P <= 64. Same outputs and
  * meaning as the per-page calls. */

@@ -1,5 +1,5 @@
-// moa_attention.hip -- ops::sliding_attention (FO/src/ops.rs:118-128): decode attention of one token
-// row over the sliding layer's ring cache.
+// moa_attention.hip -- ops::sliding_attention (FO/src/ops.rs:118-128): decode attention of token
+// rows over the sliding layer's ring cache.
 //
 // For KV head n and its query heads g = 0, 1 (FO/src/axes.rs: Ns = 8, Gs = 2, Ds = 256, Ts = 1024):
 //   s_t = q_g . k_t (scale 1.0), over the slots t whose mask value is non-zero;
@@ -12,14 +12,15 @@
 // unless masked slots hold scores far above the valid ones. Here the max is taken over the valid
 // slots only. A row with no valid slot returns zeros.
 //
-// Split over slots ("flash decoding"): workgroup (n, c, m) takes the 32 slots 32 c .. 32 c + 31
+// Few rows: split over slots ("flash decoding"): workgroup (n, c, m) takes the 32 slots 32 c .. 32 c + 31
 // of head n for token row m. It computes its partial (max, sum of exp, sum of exp * v) for both
 // query heads and publishes it with agent-scope stores. Then it adds one to the head's ticket
 // counter; the workgroup that completes the head's 32 (the counter's old value is 31 mod 32)
 // combines the partials. Nothing waits on another workgroup, so residency is not required.
 // The head is the grid's x index: workgroups go to the 8 XCDs round-robin by linear index, so all
 // 32 of head n run on XCD n and its ticket and partials never cross XCDs (7.10 -> 6.96 us per
-// call against the chunk as x index; the results do not depend on the placement).
+// call against the chunk as x index; the results do not depend on the placement). More rows:
+// attn_rows_kernel below.
 #include <hip/hip_runtime.h>
 
 #include "moa_device.h"

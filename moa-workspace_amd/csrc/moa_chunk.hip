@@ -25,7 +25,7 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kCkBlock = 256;          // four waves
+constexpr int kCkBlock = 256;          // threads of the row kernels
 constexpr int kCkBM = 256;             // rows per workgroup of the widest tile (see chunk_gemm_kernel)
 constexpr int kCkBN = 128;             // weight rows per workgroup (GeGLU: 64 up + the same 64 gate)
 constexpr int kCkBK = 64;              // k per pipeline step
@@ -118,9 +118,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t ck_rsrc(const void* base, uint
 constexpr int kCkNt = 0;
 
 // Workgroup (bx, by, bz): rows 256 by .. +256, a 128-row weight tile (columns 128 bx .. +128,
-// or for GeGLU up and gate rows 64 bx .. +64), k split bz. Wave w computes rows 64 w .. +64 of
-// the tile against all 128 weight rows: 2 x 4 blocks of v_mfma_f32_32x32x16_bf16, 128 f32
-// accumulators per lane.
+// or for GeGLU up and gate rows 64 bx .. +64), k split bz. Eight waves, two per SIMD: wave w computes rows
+// 32 w .. +32 of the tile against all 128 weight rows, 4 blocks of v_mfma_f32_32x32x16_bf16, 64 f32
+// accumulators per lane. (Four waves of 64 rows, one per SIMD, read each weight fragment from LDS half as often
+// but wait alone: FP8 layer of 256 rows 164.5 against 162.3 us, of 1000 rows 474 against 465, NVFP4 497 against 491.)
 //   Activations (A tiles) go from memory straight into the registers of the lanes that feed them
 //   to the MFMA (no other wave needs them): per 64-k step lane (l32, h) holds 32 bf16 of row l32
 //   of each 32-row block, k 32 h .. 32 h + 31, in four 1 KB-contiguous loads. MFMA j (j = 0..3)
@@ -128,23 +129,27 @@ constexpr int kCkNt = 0;
 //   permutation of the step's 64 k. Row blocks past M read zeros (the buffer ends there); rows
 //   past M are not stored.
 //   Weights (FP8) are staged once per workgroup through LDS, widened to bf16 on the way (exact for
-//   E4M3; once per workgroup instead of once per wave): each thread moves two 16-byte chunks per
-//   step, loaded eight steps ahead (HBM latency at the rate the whole chip streams weights) and
+//   E4M3; once per workgroup instead of once per wave): each thread moves one 16-byte chunk (with four waves
+//   two) per step, loaded eight steps ahead (HBM latency at the rate the whole chip streams weights) and
 //   written two steps ahead; a wave reads 64 bytes (bf16) per lane per 32-column block.
 //   All loads are buffer loads whose per-lane offsets are fixed: the step moves the scalar
 //   offset only. Prefetches past the last step repeat the last step (harmless), so the loop body
 //   has no branches.
-//   Fewer rows: RG row groups of 32 MB rows and CG = 4 / RG column groups of waves; wave (rg, cg) takes
-//   32-column blocks cg, cg + CG, .. (so that a GeGLU wave has up and gate of the same columns). BM = 32
-//   MB RG rows: 256 (RG 4, MB 2), 128 (RG 2, MB 2) or 64 (RG 2, MB 1). pick_bm chooses
-//   and has the figures.
+//   Fewer rows or weight rows, four waves: RG row groups of 32 MB rows and CG = 4 / RG column groups of waves; wave
+//   (rg, cg) takes 32-column blocks cg, cg + CG, .. (so that a GeGLU wave has up and gate of the same columns).
+//   BM = 32 MB RG rows: 256 (RG 4, MB 2; 64 weight rows only), 128 (RG 2, MB 2) or 64 (RG 2, MB 1). pick_bm
+//   chooses and has the figures.
+constexpr int ck_waves(int BN, int BM) { return BN == 128 && BM == 256 ? 8 : 4; }
+constexpr int ck_per_simd(int BN, int BM) { return BN == 64 && BM == 256 ? 1 : 2; }
+
 template <Epi E, ScaleKind SK, FfnFormat F = FfnFormat::FP8, int BN = kCkBN, int BM = kCkBM>
-__global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(BM == 256 ? 1 : 2, BM == 256 ? 1 : 2))) void chunk_gemm_kernel(GemmArgs g) {
+__global__ __launch_bounds__(64 * ck_waves(BN, BM)) __attribute__((amdgpu_waves_per_eu(ck_per_simd(BN, BM), ck_per_simd(BN, BM))))
+void chunk_gemm_kernel(GemmArgs g) {
     static_assert(BN == 128 || (BN == 64 && E == Epi::F32Partial), "128 weight rows, or 64 for split-K partials");
-    constexpr int RG = BM == 256 ? 4 : 2, MB = BM / 32 / RG, CG = 4 / RG;
+    constexpr int NW = ck_waves(BN, BM), RG = BM == 256 ? NW : 2, MB = BM / 32 / RG, CG = NW / RG;
     static_assert(BM == 256 || BM == 128 || BM == 64, "row tiles");
     constexpr int NB = BN / 32 / CG;   // 32-column blocks per wave
-    constexpr int RPT = BN / 64;  // staged weight rows per thread
+    constexpr int RPT = BN / (16 * NW);  // staged weight rows per thread
     constexpr bool FP4 = F != FfnFormat::FP8;
     // bytes per weight row and per 64-k step; FP4 block-scale bytes per row and per step
     const int rb = FP4 ? g.K / 2 : g.K;
@@ -153,7 +158,7 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(BM == 
     constexpr int kStepS = F == FfnFormat::NVFP4 ? 4 : 2;
     // three weight buffers during the loop; the GeGLU epilogue reuses the space for its transpose
     constexpr int kWsBytes = BN * kCkWStride, kTpStride = 72;
-    constexpr int kLds = 3 * kWsBytes > 4 * 64 * kTpStride * 2 ? 3 * kWsBytes : 4 * 64 * kTpStride * 2;
+    constexpr int kLds = 3 * kWsBytes > NW * 32 * MB * kTpStride * 2 ? 3 * kWsBytes : NW * 32 * MB * kTpStride * 2;
     __shared__ __attribute__((aligned(16))) uint8_t smem[kLds];
     uint8_t(*ws)[kWsBytes] = reinterpret_cast<uint8_t(*)[kWsBytes]>(smem);
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -163,7 +168,7 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(BM == 
     const int m_wave = m_blk + rg * 32 * MB;
     const int kz = g.K / gridDim.z, kbeg = blockIdx.z * kz, nsteps = kz / kCkBK;
 
-    // staged weight rows of this thread: tile row r0 (and r0 + 64 when BN = 128), k 16 q .. 16 q + 15 of each step
+    // staged weight rows of this thread: tile row r0 (and, four waves on BN = 128, r0 + 64), k 16 q .. 16 q + 15 of each step
     // (FP8: 16 bytes; FP4: 8 bytes of codes and the one block-scale code covering them)
     const int r0 = t >> 2, q = t & 3;
     __amdgpu_buffer_rsrc_t wrs[2], srs[2];
@@ -175,12 +180,14 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(BM == 
         const size_t off = (size_t)blockIdx.x * 64 * rb;
         wrs[0] = ck_rsrc(g.w[0] + off, 64u * rb);
         wrs[1] = ck_rsrc(g.w2 + off, 64u * rb);
-        wvo[0] = wvo[1] = r0 * rb + kcol;
+        if (NW == 8 && __builtin_amdgcn_readfirstlane(wave) >= 4) wrs[0] = wrs[1];  // waves 4 .. 7 stage the gate rows
+        wvo[0] = wvo[1] = (r0 & 63) * rb + kcol;
         if constexpr (FP4) {
             const size_t so = (size_t)blockIdx.x * 64 * sb;
             srs[0] = ck_rsrc(g.wsc[0] + so, 64u * sb);
             srs[1] = ck_rsrc(g.wsc2 + so, 64u * sb);
-            svo[0] = svo[1] = r0 * sb + scol;
+            if (NW == 8 && __builtin_amdgcn_readfirstlane(wave) >= 4) srs[0] = srs[1];
+            svo[0] = svo[1] = (r0 & 63) * sb + scol;
         }
     } else {
         const int n0 = blockIdx.x * BN;
@@ -282,17 +289,13 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(BM == 
     load_w(wr[1], WD + 1);
     __syncthreads();
     read_b(bb[0], 0, 0);
+    // Four fragments per step (eight waves, two per SIMD). Each fragment's LDS reads go out during the one
+    // before; the A prefetch rides with fragment 0, the weight staging with fragment 1.
     [[maybe_unused]] auto body4 = [&](auto P, int s) {
         constexpr int c = decltype(P)::value;  // s mod 6
         constexpr int cb = c % 3, nbuf = (c + 1) % 3;
         const uint4(&a)[MB][4] = ar[c % 3];
-        // Fences fix the issue order: each fragment's LDS reads go out during the previous
-        // fragment's eight MFMAs, one or two other instructions after each MFMA (a single wave
-        // per SIMD issues them while the MFMA runs); the A prefetch rides with fragment 0, the
-        // weight staging (16 widenings, 4 LDS writes, 2 loads) with fragment 1.
         constexpr int kDsR = 0x100, kDsW = 0x200, kVmR = 0x020, kValu = 0x002, kMfma = 0x008;
-        constexpr int kWLoads = FP4 ? 4 : 2;                    // weight (and scale) loads per step
-        constexpr int kWValu = F == FfnFormat::NVFP4 ? 8 : 2;   // widening instructions per MFMA slot
         read_b(bb[1], cb, 1);
         load_a(ar[(c + 2) % 3], s + 2);
         mfma8(a, bb[0], Par<0>{});
@@ -300,11 +303,7 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(BM == 
         for (int i = 0; i < 4; ++i) {
             __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
             __builtin_amdgcn_sched_group_barrier(kDsR, 1, 0);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(kVmR, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(kVmR, 1, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
         read_b(bb[0], cb, 2);
@@ -315,15 +314,9 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(BM == 
         for (int i = 0; i < 4; ++i) {
             __builtin_amdgcn_sched_group_barrier(kMfma, 1, 1);
             __builtin_amdgcn_sched_group_barrier(kDsR, 1, 1);
-            __builtin_amdgcn_sched_group_barrier(kValu, kWValu, 1);
+            __builtin_amdgcn_sched_group_barrier(kValu, F == FfnFormat::NVFP4 ? 8 : 2, 1);
         }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 1);
-            __builtin_amdgcn_sched_group_barrier(kValu, kWValu, 1);
-            __builtin_amdgcn_sched_group_barrier(kDsW, 1, 1);
-        }
-        __builtin_amdgcn_sched_group_barrier(kVmR, kWLoads, 1);
+        __builtin_amdgcn_sched_group_barrier(kDsW, 2, 1);
         __builtin_amdgcn_sched_barrier(0);
         read_b(bb[1], cb, 3);
         mfma8(a, bb[0], Par<2>{});
@@ -332,7 +325,6 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(BM == 
             __builtin_amdgcn_sched_group_barrier(kMfma, 1, 2);
             __builtin_amdgcn_sched_group_barrier(kDsR, 1, 2);
         }
-        __builtin_amdgcn_sched_group_barrier(kMfma, 4, 2);
         __builtin_amdgcn_sched_barrier(0);
         read_b(bb[0], nbuf, 0);
         mfma8(a, bb[1], Par<3>{});
@@ -341,11 +333,10 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(BM == 
             __builtin_amdgcn_sched_group_barrier(kMfma, 1, 3);
             __builtin_amdgcn_sched_group_barrier(kDsR, 1, 3);
         }
-        __builtin_amdgcn_sched_group_barrier(kMfma, 4, 3);
+        __builtin_amdgcn_sched_barrier(0);
         // Step barrier. Every read of the buffer the next step overwrites fed an MFMA of this step
         // (so it is complete); the next step's buffer needs this wave's LDS writes complete, and
         // only the four reads just issued may still be in flight: lgkmcnt(4), not 0.
-        __builtin_amdgcn_sched_barrier(0);
         __asm__ volatile("s_waitcnt lgkmcnt(4)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         __asm__ volatile("" ::: "memory");
@@ -465,7 +456,7 @@ __global__ __launch_bounds__(kCkBlock) __attribute__((amdgpu_waves_per_eu(BM == 
         // p = bf16(gelu(gate) * up) for the wave's 64 rows x 64 columns, transposed through the
         // wave's own 9 KB of LDS (row stride 72 elements) so that each lane then stores whole
         // 16-byte units of the A tiles (row, 8 consecutive columns).
-        uint16_t* tp = reinterpret_cast<uint16_t*>(smem) + wave * (64 * kTpStride);
+        uint16_t* tp = reinterpret_cast<uint16_t*>(smem) + wave * (32 * MB * kTpStride);
         // the format's commit of each projection: FP8 bf16(sum * s[n]); NVFP4 bf16(bf16(sum) * 1/g);
         // MXFP4 bf16(sum) (generate_references.py:265-274, 358-372)
         const float gu = F == FfnFormat::NVFP4 ? *g.g0 : 1.0f, gg = F == FfnFormat::NVFP4 ? *g.g2 : 1.0f;
@@ -771,12 +762,12 @@ int pick_splits(int tiles, int ksteps, size_t rows_x_cols) {
     return sp;
 }
 
-// Weight rows per workgroup of a split-K projection. The O projection (K = 4096) takes 64: twice
-// the tiles of 128-row tiles, so half the k splits fill the device and half the f32 partial sums
-// are written and read back (measured at M = 256: GEMM 17.3 -> 16.5 us, post rows 9.1 -> 6.9 us).
-// QKV takes 64 up to 256 rows (launch_qkv_chunk). Down keeps 128, whose main loop does twice the
-// MFMA work per A load and per barrier (with 64, down measured 39.1 -> 44.6 us against 9.5 ->
-// 7.1 us saved in its post rows).
+// Weight rows per workgroup of a split-K projection: 64 where twice the tiles of 128-row tiles fill the device
+// with half the k splits, so half the f32 partial sums are written and read back: O up to 256 rows (at 256:
+// GEMM 17.3 -> 16.5 us, post rows 9.1 -> 6.9), QKV up to 128. Else 128, whose main loop does twice the MFMA
+// work per A load and per barrier, on eight waves for 256-row tiles: QKV of a 200-row full-attention layer (with O)
+// 72.6 -> 66.0 us, the 200-row FP8 layer 153 -> 150, 256 rows even; O at 1000 rows 484 -> 479 (layer). Down always
+// takes 128 (with 64, down measured 39.1 -> 44.6 us against 9.5 -> 7.1 us saved in its post rows).
 constexpr int kCkOBN = 64;
 
 // Rows per workgroup of a call of M rows: the smallest row tile that holds them, so that no wave computes
@@ -793,7 +784,9 @@ hipError_t gemm_launch(const GemmArgs& g, int splits, int bm, hipStream_t s) {
     switch (bm) {
         case 64: return ck_launch(chunk_gemm_kernel<E, SK, F, BN, 64>, grid, s, g);
         case 128: return ck_launch(chunk_gemm_kernel<E, SK, F, BN, 128>, grid, s, g);
-        case kCkBM: return ck_launch(chunk_gemm_kernel<E, SK, F, BN, kCkBM>, grid, s, g);
+        case kCkBM:
+            hipLaunchKernelGGL((chunk_gemm_kernel<E, SK, F, BN, kCkBM>), grid, dim3(64 * ck_waves(BN, kCkBM)), 0, s, g);
+            return hipGetLastError();
     }
     return hipErrorInvalidValue;
 }
@@ -844,11 +837,8 @@ hipError_t launch_qkv_chunk(const QkvParams& p, int m0, int M, hipStream_t s, De
     g.w[0] = p.qw; g.w[1] = p.kw; g.w[2] = p.vw;
     g.nseg[0] = 0; g.nseg[1] = kQs; g.nseg[2] = kQs + kPs; g.nseg[3] = kQkvRowsTotal; g.nsegs = 3;
     g.yf = ctx->fbuf;
-    // Up to 256 rows, 64-row weight tiles (128 tiles x 2 k splits instead of 64 x 4: half the
-    // partial sums; M = 256: 39.3 -> 37.4 us). Beyond, they would not split, and the 512 tiles
-    // of M = 1024 measured 112 us against 102 with 128-row tiles.
     const int bm = pick_bm(M), mt = m_tiles(M, bm);
-    const bool narrow = M <= 256;
+    const bool narrow = M <= 128;
     const int sp = pick_splits(kQkvRowsTotal / (narrow ? kCkOBN : kCkBN) * mt, kH / kCkBK, (size_t)M * kQkvRowsTotal);
     e = narrow ? gemm_partial<FfnFormat::FP8, kCkOBN>(g, sp, bm, s) : gemm_partial(g, sp, bm, s);
     if (e != hipSuccess) return e;
@@ -858,7 +848,7 @@ hipError_t launch_qkv_chunk(const QkvParams& p, int m0, int M, hipStream_t s, De
 
 // full_project_qkv: the rows once through the GEMM over [Wq; Wk], then the head kernel of the rows
 // path. (Called 16 rows at a time, the rows path reads the weights every 16 rows: QKV and O of 300 rows take
-// 610 us that way, 98 us this way.)
+// 610 us that way, 93 us this way.)
 hipError_t launch_full_qkv_chunk(const QkvParams& p, int m0, int M, hipStream_t s, DevCtx* ctx) {
     constexpr int N = kQf + kPf;
     hipError_t e = ck_launch(chunk_rmsnorm_rows_kernel<true>, dim3(M), s, p.x + (size_t)m0 * kH, p.in_rms, ctx->hbuf);
@@ -869,7 +859,7 @@ hipError_t launch_full_qkv_chunk(const QkvParams& p, int m0, int M, hipStream_t 
     g.nseg[0] = 0; g.nseg[1] = kQf; g.nseg[2] = N; g.nsegs = 2;
     g.yf = ctx->fbuf;
     const int bm = pick_bm(M), mt = m_tiles(M, bm);
-    const bool narrow = M <= 256;  // as launch_qkv_chunk
+    const bool narrow = M <= 128;  // as launch_qkv_chunk
     const int sp = pick_splits(N / (narrow ? kCkOBN : kCkBN) * mt, kH / kCkBK, (size_t)M * N);
     e = narrow ? gemm_partial<FfnFormat::FP8, kCkOBN>(g, sp, bm, s) : gemm_partial(g, sp, bm, s);
     if (e != hipSuccess) return e;
@@ -888,9 +878,10 @@ static hipError_t o_chunk_gemm(const OParams& p, int m0, int M, hipStream_t s, D
     g.x = ctx->pbuf; g.M = M; g.N = kH; g.K = K;
     g.w[0] = p.ow; g.nseg[0] = 0; g.nseg[1] = kH; g.nsegs = 1;
     g.yf = ctx->fbuf;
-    const int bm = pick_bm(M);
-    *sp = pick_splits(kH / kCkOBN * m_tiles(M, bm), K / kCkBK, (size_t)M * kH);
-    return gemm_partial<FfnFormat::FP8, kCkOBN>(g, *sp, bm, s);
+    const int bm = pick_bm(M), mt = m_tiles(M, bm);
+    const bool narrow = M <= 256;
+    *sp = pick_splits(kH / (narrow ? kCkOBN : kCkBN) * mt, K / kCkBK, (size_t)M * kH);
+    return narrow ? gemm_partial<FfnFormat::FP8, kCkOBN>(g, *sp, bm, s) : gemm_partial(g, *sp, bm, s);
 }
 
 hipError_t launch_o_chunk(const OParams& p, int m0, int M, hipStream_t s, DevCtx* ctx) {

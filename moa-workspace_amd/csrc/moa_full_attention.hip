@@ -14,7 +14,7 @@
 // RNGD kernel takes its page max over every slot, rounds scores and weights to bf16 and adds 1e-6
 // to each page sum, which moves results within rounding.
 //
-// Two launches per page:
+// Two launches per page for up to 16 rows (for more, fattn_rows_kernel below takes the first's place):
 //  1. fattn_partial_kernel, grid (8 slot chunks, 4 dim blocks, M): workgroup (c, b, m) scores the
 //     64 slots of chunk c against all 16 heads on the matrix cores (v_mfma_f32_16x16x32_bf16: the
 //     heads as A rows, K rows as B columns, each wave a quarter of the 512 dims), takes each
@@ -25,12 +25,13 @@
 //  2. fattn_combine_kernel, grid (16 heads, M): merges the 8 chunks with the old state and writes
 //     the new one. One workgroup owns a head's state, so no other reads it while it is replaced.
 //
-// moa_full_attention computes the same state over pages 0 .. P - 1 in two launches instead of 2 P:
+// moa_full_attention computes the same state over pages 0 .. P - 1 in two launches instead of 2 P (more where
+// the rows' records would not fit the scratch); with few rows times pages:
 // the partial pass runs over every page at once -- up to 8 pages with the dim-split kernel (one
 // chunk per workgroup), beyond with fattn_span_kernel (a workgroup takes a span of chunks over all
 // dims with an online softmax; at most 256 records per row) -- and fattn_merge_kernel merges the
 // records with a grid of (16 heads, 8 dim blocks): no old state is read, so the split is free of
-// races.
+// races. With more, fattn_rows_kernel shares every tile of K and V among four token rows.
 #include <hip/hip_runtime.h>
 
 #include "moa_device.h"
