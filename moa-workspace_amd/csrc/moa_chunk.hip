@@ -135,18 +135,22 @@ constexpr int kCkNt = 0;
 //   All loads are buffer loads whose per-lane offsets are fixed: the step moves the scalar
 //   offset only. Prefetches past the last step repeat the last step (harmless), so the loop body
 //   has no branches.
-//   Fewer rows or weight rows, four waves: RG row groups of 32 MB rows and CG = 4 / RG column groups of waves; wave
-//   (rg, cg) takes 32-column blocks cg, cg + CG, .. (so that a GeGLU wave has up and gate of the same columns).
-//   BM = 32 MB RG rows: 256 (RG 4, MB 2; 64 weight rows only), 128 (RG 2, MB 2) or 64 (RG 2, MB 1). pick_bm
-//   chooses and has the figures.
-constexpr int ck_waves(int BN, int BM) { return BN == 128 && BM == 256 ? 8 : 4; }
+//   Fewer rows: waves in RG groups of 32 MB rows, CG column groups and, for 64 rows, KG = 2 k groups, of which
+//   wave (kg, rg, cg) takes 32-column blocks cg, cg + CG, .. (so that a GeGLU wave has up and gate of the same
+//   columns) and of each step's MFMAs j 2 kg and 2 kg + 1; the k groups' sums meet in LDS at the end. Always eight
+//   waves (four before, one per SIMD: FP8 / NVFP4 layer of 128 rows 123 / 130 -> 118 / 121 us, of 64 rows 99.6 /
+//   104 -> 98.0 / 99.5, of 17 rows 90.2 / 99 -> 88.5 / 92; full-attention QKV and O of 100 rows 59 -> 49), except
+//   with 64 weight rows: four. pick_bm chooses the rows and has the figures. A loads deeper than two steps gained
+//   nothing. At 17 rows a GeGLU step waits for weights (all loads from one step: 31 -> 20 us, 18 without widening).
+constexpr int ck_waves(int BN, int BM) { return BN == 128 ? 8 : 4; }
 constexpr int ck_per_simd(int BN, int BM) { return BN == 64 && BM == 256 ? 1 : 2; }
 
 template <Epi E, ScaleKind SK, FfnFormat F = FfnFormat::FP8, int BN = kCkBN, int BM = kCkBM>
 __global__ __launch_bounds__(64 * ck_waves(BN, BM)) __attribute__((amdgpu_waves_per_eu(ck_per_simd(BN, BM), ck_per_simd(BN, BM))))
 void chunk_gemm_kernel(GemmArgs g) {
     static_assert(BN == 128 || (BN == 64 && E == Epi::F32Partial), "128 weight rows, or 64 for split-K partials");
-    constexpr int NW = ck_waves(BN, BM), RG = BM == 256 ? NW : 2, MB = BM / 32 / RG, CG = NW / RG;
+    constexpr int NW = ck_waves(BN, BM), MB = BN == 64 && BM == 256 ? 2 : 1, RG = BM / 32 / MB;
+    constexpr int KG = BN == 128 && BM == 64 ? 2 : 1, CG = NW / RG / KG, JN = 4 / KG;  // JN: MFMAs per block and step
     static_assert(BM == 256 || BM == 128 || BM == 64, "row tiles");
     constexpr int NB = BN / 32 / CG;   // 32-column blocks per wave
     constexpr int RPT = BN / (16 * NW);  // staged weight rows per thread
@@ -163,7 +167,7 @@ void chunk_gemm_kernel(GemmArgs g) {
     uint8_t(*ws)[kWsBytes] = reinterpret_cast<uint8_t(*)[kWsBytes]>(smem);
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int hf = lane >> 5, l32 = lane & 31;
-    const int rg = wave / CG, cg = wave % CG;
+    const int kg = wave / (RG * CG), rg = wave / CG % RG, cg = wave % CG;
     const int m_blk = blockIdx.y * BM;
     const int m_wave = m_blk + rg * 32 * MB;
     const int kz = g.K / gridDim.z, kbeg = blockIdx.z * kz, nsteps = kz / kCkBK;
@@ -208,7 +212,7 @@ void chunk_gemm_kernel(GemmArgs g) {
     const __amdgpu_buffer_rsrc_t ars = ck_rsrc(g.x + (size_t)(m_blk >> 5) * kst * 2048, (uint32_t)rblks * kst * 4096u);
     int avo[MB];
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) avo[mb] = ((rg * MB + mb) * kst * 2048 + lane * 8) * 2 + (kbeg / kCkBK) * 4096;
+    for (int mb = 0; mb < MB; ++mb) avo[mb] = ((rg * MB + mb) * kst * 2048 + lane * 8) * 2 + (kbeg / kCkBK) * 4096 + kg * JN * 1024;
 
     f32x16 acc[MB][NB];
 #pragma unroll
@@ -220,8 +224,8 @@ void chunk_gemm_kernel(GemmArgs g) {
 
     constexpr int WD = 6;  // weight register sets: W(s + 2) is loaded six steps before it is staged
     uint4 wr[WD][2];       // [set][row pair]
-    uint4 ar[3][MB][4];    // [set][32-row block][16 bytes]: A(s) in set s mod 3, loaded two steps ahead
-    bf16x8 bb[2][4];       // B fragments: [set][MFMA j]
+    uint4 ar[3][MB][JN];   // [set][32-row block][16 bytes]: A(s) in set s mod 3, loaded two steps ahead
+    bf16x8 bb[2][JN];      // B fragments: [set][MFMA j]
     const int last = nsteps - 1;
     // FP4: .x, .y the 16 codes, .z the block-scale code
     auto load_w = [&](uint4 (&dst)[2], int s) {
@@ -253,23 +257,23 @@ void chunk_gemm_kernel(GemmArgs g) {
             }
         }
     };
-    auto load_a = [&](uint4 (&dst)[MB][4], int s) {
+    auto load_a = [&](uint4 (&dst)[MB][JN], int s) {
         const int so = min(s, last) * 4096;
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < JN; ++i)
                 dst[mb][i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ars, avo[mb] + 1024 * i, so, 0));
     };
-    auto read_b = [&](bf16x8 (&dst)[4], int buf, int nb) {
-        const bf16x8* bp = reinterpret_cast<const bf16x8*>(&ws[buf][(32 * (cg + CG * nb) + l32) * kCkWStride + 64 * hf]);
+    auto read_b = [&](bf16x8 (&dst)[JN], int buf, int nb) {
+        const bf16x8* bp = reinterpret_cast<const bf16x8*>(&ws[buf][(32 * (cg + CG * nb) + l32) * kCkWStride + 64 * hf + 16 * JN * kg]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) dst[j] = bp[j];
+        for (int j = 0; j < JN; ++j) dst[j] = bp[j];
     };
-    auto mfma8 = [&](const uint4 (&a)[MB][4], const bf16x8 (&b)[4], auto NBI) {
+    auto mfma8 = [&](const uint4 (&a)[MB][JN], const bf16x8 (&b)[JN], auto NBI) {
         constexpr int nb = decltype(NBI)::value;
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < JN; ++j)
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb)
                 acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a[mb][j]), b[j], acc[mb][nb], 0, 0, 0);
@@ -294,7 +298,7 @@ void chunk_gemm_kernel(GemmArgs g) {
     [[maybe_unused]] auto body4 = [&](auto P, int s) {
         constexpr int c = decltype(P)::value;  // s mod 6
         constexpr int cb = c % 3, nbuf = (c + 1) % 3;
-        const uint4(&a)[MB][4] = ar[c % 3];
+        const uint4(&a)[MB][JN] = ar[c % 3];
         constexpr int kDsR = 0x100, kDsW = 0x200, kVmR = 0x020, kValu = 0x002, kMfma = 0x008;
         read_b(bb[1], cb, 1);
         load_a(ar[(c + 2) % 3], s + 2);
@@ -346,11 +350,11 @@ void chunk_gemm_kernel(GemmArgs g) {
     // W(s + 2)) beside fragment 1's LDS reads; fragment 1 the A and weight prefetches and, last of
     // the step's LDS operations, the next step's first fragment -- so lgkmcnt(4) at the barrier
     // still leaves every LDS write of this wave complete.
-    constexpr int kMf = 4 * MB;  // MFMAs per fragment
+    constexpr int kMf = JN * MB;  // MFMAs per fragment
     [[maybe_unused]] auto body2 = [&](auto P, int s) {
         constexpr int c = decltype(P)::value;  // s mod 6
         constexpr int cb = c % 3, nbuf = (c + 1) % 3;
-        const uint4(&a)[MB][4] = ar[c % 3];
+        const uint4(&a)[MB][JN] = ar[c % 3];
         constexpr int kDsR = 0x100, kDsW = 0x200, kVmR = 0x020, kValu = 0x002, kMfma = 0x008;
         constexpr int kWLoads = (FP4 ? 2 : 1) * RPT;
         constexpr int kWValu = (F == FfnFormat::NVFP4 ? 4 : 1) * RPT * 8 / kMf;
@@ -386,7 +390,8 @@ void chunk_gemm_kernel(GemmArgs g) {
         }
         __builtin_amdgcn_sched_group_barrier(kVmR, kWLoads, 1);
         __builtin_amdgcn_sched_barrier(0);
-        __asm__ volatile("s_waitcnt lgkmcnt(4)" ::: "memory");
+        if constexpr (JN == 2) __asm__ volatile("s_waitcnt lgkmcnt(2)" ::: "memory");
+        else __asm__ volatile("s_waitcnt lgkmcnt(4)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         __asm__ volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
@@ -396,7 +401,7 @@ void chunk_gemm_kernel(GemmArgs g) {
     [[maybe_unused]] auto body1 = [&](auto P, int s) {
         constexpr int c = decltype(P)::value;  // s mod 6
         constexpr int nbuf = (c + 1) % 3;
-        const uint4(&a)[MB][4] = ar[c % 3];
+        const uint4(&a)[MB][JN] = ar[c % 3];
         constexpr int kDsR = 0x100, kMfma = 0x008;
         store_w(wr[(c + 2) % WD], (c + 2) % 3);
         load_a(ar[(c + 2) % 3], s + 2);
@@ -435,7 +440,25 @@ void chunk_gemm_kernel(GemmArgs g) {
     if (s < nsteps) body(Par<3>{}, s++);
     if (s < nsteps) body(Par<4>{}, s++);
 
-    if constexpr (E == Epi::GeGLU) __syncthreads();  // the loop's LDS reads are done: the transpose may reuse it
+    // The loop's LDS reads are done: the k groups' sums and the transpose may reuse it.
+    constexpr int kRedBytes = KG == 2 ? RG * CG * NB * 4096 : 0;
+    static_assert(kRedBytes + RG * CG * 32 * MB * kTpStride * 2 <= kLds, "the k groups' sums and the transposes");
+    if constexpr (E == Epi::GeGLU || KG == 2) __syncthreads();
+    if constexpr (KG == 2) {
+        float* red = reinterpret_cast<float*>(smem) + (rg * CG + cg) * NB * 1024 + lane;
+        if (kg == 1) {
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) red[(nb * 16 + r) * 64] = acc[0][nb][r];
+        }
+        __syncthreads();
+        if (kg == 1) return;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[0][nb][r] += red[(nb * 16 + r) * 64];
+    }
     if (m_wave >= g.M) return;
     // Accumulator element r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4 of the 32-row block,
     // column l % 32 of the 32-column block. A wave whose 64 rows all lie below M stores without
@@ -456,7 +479,7 @@ void chunk_gemm_kernel(GemmArgs g) {
         // p = bf16(gelu(gate) * up) for the wave's 64 rows x 64 columns, transposed through the
         // wave's own 9 KB of LDS (row stride 72 elements) so that each lane then stores whole
         // 16-byte units of the A tiles (row, 8 consecutive columns).
-        uint16_t* tp = reinterpret_cast<uint16_t*>(smem) + wave * (32 * MB * kTpStride);
+        uint16_t* tp = reinterpret_cast<uint16_t*>(smem + kRedBytes) + (rg * CG + cg) * (32 * MB * kTpStride);
         // the format's commit of each projection: FP8 bf16(sum * s[n]); NVFP4 bf16(bf16(sum) * 1/g);
         // MXFP4 bf16(sum) (generate_references.py:265-274, 358-372)
         const float gu = F == FfnFormat::NVFP4 ? *g.g0 : 1.0f, gg = F == FfnFormat::NVFP4 ? *g.g2 : 1.0f;
@@ -778,15 +801,19 @@ int pick_bm(int M) { return M <= 64 ? 64 : (M <= 128 ? 128 : kCkBM); }
 
 int m_tiles(int M, int bm) { return (M + bm - 1) / bm; }
 
+template <Epi E, ScaleKind SK, FfnFormat F, int BN, int BM>
+hipError_t gemm_launch_bm(const GemmArgs& g, int splits, hipStream_t s) {
+    const dim3 grid(g.N / (E == Epi::GeGLU ? 64 : BN), m_tiles(g.M, BM), splits);
+    hipLaunchKernelGGL((chunk_gemm_kernel<E, SK, F, BN, BM>), grid, dim3(64 * ck_waves(BN, BM)), 0, s, g);
+    return hipGetLastError();
+}
+
 template <Epi E, ScaleKind SK, FfnFormat F, int BN>
 hipError_t gemm_launch(const GemmArgs& g, int splits, int bm, hipStream_t s) {
-    const dim3 grid(g.N / (E == Epi::GeGLU ? 64 : BN), m_tiles(g.M, bm), splits);
     switch (bm) {
-        case 64: return ck_launch(chunk_gemm_kernel<E, SK, F, BN, 64>, grid, s, g);
-        case 128: return ck_launch(chunk_gemm_kernel<E, SK, F, BN, 128>, grid, s, g);
-        case kCkBM:
-            hipLaunchKernelGGL((chunk_gemm_kernel<E, SK, F, BN, kCkBM>), grid, dim3(64 * ck_waves(BN, kCkBM)), 0, s, g);
-            return hipGetLastError();
+        case 64: return gemm_launch_bm<E, SK, F, BN, 64>(g, splits, s);
+        case 128: return gemm_launch_bm<E, SK, F, BN, 128>(g, splits, s);
+        case kCkBM: return gemm_launch_bm<E, SK, F, BN, kCkBM>(g, splits, s);
     }
     return hipErrorInvalidValue;
 }
