@@ -800,9 +800,11 @@ int pick_splits(int tiles, int ksteps, size_t rows_x_cols) {
 // Weight rows per workgroup of a split-K projection: 64 where twice the tiles of 128-row tiles fill the device
 // with half the k splits, so half the f32 partial sums are written and read back: O up to 256 rows (at 256:
 // GEMM 17.3 -> 16.5 us, post rows 9.1 -> 6.9), QKV up to 128. Else 128, whose main loop does twice the MFMA
-// work per A load and per barrier, on eight waves for 256-row tiles: QKV of a 200-row full-attention layer (with O)
+// work per A load and per barrier, on eight waves: QKV of a 200-row full-attention layer (with O)
 // 72.6 -> 66.0 us, the 200-row FP8 layer 153 -> 150, 256 rows even; O at 1000 rows 484 -> 479 (layer). Down always
-// takes 128 (with 64, down measured 39.1 -> 44.6 us against 9.5 -> 7.1 us saved in its post rows).
+// takes 128 (with 64, down measured 39.1 -> 44.6 us against 9.5 -> 7.1 us saved in its post rows), and so does the
+// full-attention QKV, whose 136 tiles of 64 rows would not split: with O, 20 rows 38.9 -> 37.1 us, 64 rows 44.8 ->
+// 40.2, 128 rows 52.5 -> 50.0 (the sliding QKV's 128 tiles do: 17..128 rows 0.3-1 us faster with 64).
 constexpr int kCkOBN = 64;
 
 // Rows per workgroup of a call of M rows: the smallest row tile that holds them, so that no wave computes
@@ -898,9 +900,8 @@ hipError_t launch_full_qkv_chunk(const QkvParams& p, int m0, int M, hipStream_t 
     g.nseg[0] = 0; g.nseg[1] = kQf; g.nseg[2] = N; g.nsegs = 2;
     g.yf = ctx->fbuf;
     const int bm = pick_bm(M), mt = m_tiles(M, bm);
-    const bool narrow = M <= 128;  // as launch_qkv_chunk
-    const int sp = pick_splits(N / (narrow ? kCkOBN : kCkBN) * mt, kH / kCkBK, (size_t)M * N);
-    e = narrow ? gemm_partial<FfnFormat::FP8, kCkOBN>(g, sp, bm, s) : gemm_partial(g, sp, bm, s);
+    const int sp = pick_splits(N / kCkBN * mt, kH / kCkBK, (size_t)M * N);
+    e = gemm_partial(g, sp, bm, s);
     if (e != hipSuccess) return e;
     return launch_full_qkv_heads(p, m0, M, ctx->fbuf, sp, s, ctx);
 }
