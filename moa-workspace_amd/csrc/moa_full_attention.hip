@@ -659,19 +659,23 @@ __global__ __launch_bounds__(kFrBlock) __attribute__((amdgpu_waves_per_eu(2, 2))
 }
 
 // Workgroup (h, m) merges head h's nrec (at most 8) records into the row's state; thread t owns dims
-// 2 t, 2 t + 1.
-__global__ __launch_bounds__(kFaBlock) void fattn_combine_kernel(const float* __restrict__ part, int nrec, float* rmax,
-                                                                 float* rsum, uint16_t* out, int first) {
+// 2 t, 2 t + 1. All: nrec is 8, known to the compiler, so that every address is at a fixed offset (three one-row
+// pages as a graph: 24.2 us, with the count as an argument 24.75).
+template <bool All>
+__global__ __launch_bounds__(kFaBlock) void fattn_combine_kernel(const float* __restrict__ part, float* rmax,
+                                                                 float* rsum, uint16_t* out, int first, int n) {
     const int h = blockIdx.x, m = blockIdx.y, t = threadIdx.x;
+    const int nrec = All ? kFaChunks : n;
     const float* pm = part + (size_t)m * nrec * kFaRec;
     float mc[kFaChunks], lc[kFaChunks];
     float2 oc[kFaChunks];
 #pragma unroll
     for (int c = 0; c < kFaChunks; ++c) {
-        const float* rec = pm + min(c, nrec - 1) * kFaRec;
-        mc[c] = c < nrec ? rec[h] : -INFINITY;
-        lc[c] = rec[kGf + h];
-        oc[c] = *reinterpret_cast<const float2*>(rec + 2 * kGf + h * kDf + 2 * t);
+        const int at = (All ? c : min(c, nrec - 1)) * kFaRec;
+        mc[c] = pm[at + h];
+        if (!All && c >= nrec) mc[c] = -INFINITY;
+        lc[c] = pm[at + kGf + h];
+        oc[c] = *reinterpret_cast<const float2*>(pm + at + 2 * kGf + h * kDf + 2 * t);
     }
     const size_t sh = (size_t)m * kGf + h;
     uint32_t* op = reinterpret_cast<uint32_t*>(out + sh * kDf) + t;
@@ -771,12 +775,19 @@ __global__ __launch_bounds__(kFaBlock) void fattn_merge_kernel(const float* __re
 
 }  // namespace
 
+static hipError_t combine_rows(const float* part, int nrec, float* rmax, float* rsum, uint16_t* out, bool first, int mm,
+                               hipStream_t s) {
+    const dim3 grid(kGf, mm), block(kFaBlock);
+    if (nrec == kFaChunks) hipLaunchKernelGGL(fattn_combine_kernel<true>, grid, block, 0, s, part, rmax, rsum, out, first ? 1 : 0, nrec);
+    else hipLaunchKernelGGL(fattn_combine_kernel<false>, grid, block, 0, s, part, rmax, rsum, out, first ? 1 : 0, nrec);
+    return hipGetLastError();
+}
+
 // Rows m0 .. m0 + mm - 1 of the merge; P pages in nrec records per row.
 static hipError_t merge_rows(const float* part, int nrec, float* rmax, float* rsum, uint16_t* out, int mm, hipStream_t s) {
     const dim3 grid(kGf, kDf / kFmDims, mm), block(kFaBlock);
-    if (nrec <= kFaChunks)  // few records: a workgroup per head
-        hipLaunchKernelGGL(fattn_combine_kernel, dim3(kGf, mm), block, 0, s, part, nrec, rmax, rsum, out, 1);
-    else if (nrec <= 4 * kFmGroups) hipLaunchKernelGGL(fattn_merge_kernel<4>, grid, block, 0, s, part, nrec, rmax, rsum, out);
+    if (nrec <= kFaChunks) return combine_rows(part, nrec, rmax, rsum, out, true, mm, s);  // few: a workgroup per head
+    if (nrec <= 4 * kFmGroups) hipLaunchKernelGGL(fattn_merge_kernel<4>, grid, block, 0, s, part, nrec, rmax, rsum, out);
     else if (nrec <= 8 * kFmGroups) hipLaunchKernelGGL(fattn_merge_kernel<8>, grid, block, 0, s, part, nrec, rmax, rsum, out);
     else hipLaunchKernelGGL(fattn_merge_kernel<kFaMaxRecords / kFmGroups>, grid, block, 0, s, part, nrec, rmax, rsum, out);
     return hipGetLastError();
@@ -854,10 +865,8 @@ hipError_t launch_full_attention_page(const uint16_t* q, const uint16_t* k_page,
                                ctx->fattn_part);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(fattn_combine_kernel, dim3(kGf, mm), dim3(kFaBlock), 0, s, (const float*)ctx->fattn_part, r.nrec,
-                           running_max + (size_t)m0 * kGf, running_sum + (size_t)m0 * kGf, out + (size_t)m0 * kQf,
-                           first ? 1 : 0);
-        e = hipGetLastError();
+        e = combine_rows(ctx->fattn_part, r.nrec, running_max + (size_t)m0 * kGf, running_sum + (size_t)m0 * kGf,
+                         out + (size_t)m0 * kQf, first, mm, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
