@@ -390,11 +390,13 @@ constexpr int kFrPStride = kFaChunk + 8;        // LDS row of the weights, in el
 // (64 accumulators a lane) is rescaled only when the maximum has grown by more. The state is brought to
 // the maximum at the end.
 constexpr float kFrSlack = 8.0f;
-// From these row x pages products of a call over all pages (rows of a one-page call) on this path is used.
-// All pages, this path against the one-row kernels on every row: M x P = 2 x 4 13.5 / 9.9 us, 4 x 3 15.4 /
-// 15.4, 2 x 8 15.1 / 15.8, 16 x 1 15.9 / 16.5, 2 x 12 17.2 / 15.6, 3 x 8 17.1 / 21.7, 13 x 3 19.2 / 34.0, 2 x 64
-// 25.1 / 37.0, 200 x 6 54 / 839. One page: up to 16 rows one launch of the one-row kernel (15 us); more would be
-// several (64 rows 22.0 / 59.2, 200 rows 27 / 191).
+// From these row x pages products of a call over all pages (rows of a one-page call) on this path is used, unless
+// the span kernel takes all rows with one workgroup per CU. This path against the one-row kernels on every row
+// (us, calls replayed as a graph): M x P = 2 x 8 14.9 / 16.3, 3 x 6 15.8 / 22.4, 4 x 4 15.8 / 17.8, 8 x 2 15.8 / 20.1,
+// 16 x 1 15.7 / 25.2, 13 x 3 19.2 / 34.0, 200 x 6 50 / 1200, and host-driven 2 x 4 13.5 / 9.9. Against spans, one
+// workgroup per CU: 1 x 16 15.7 / 13.4, 1 x 64 22.5 / 20.7, 2 x 9 16.5 / 13.8, 2 x 16 17.9 / 15.9, 3 x 9 19.3 / 16.3;
+// more: 3 x 12 20.3 / 26.9, 2 x 24 19.0 / 28.2, 4 x 10 21.6 / 28.4, 2 x 64 25.0 / 41.0. One page: up to 16 rows one
+// launch of the one-row kernel (15 us); more would be several (64 rows 22.0 / 59.2, 200 rows 27 / 191).
 constexpr int kFrMinRowPages = 16;
 constexpr int kFrMinPageRows = 17;
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -659,8 +661,7 @@ __global__ __launch_bounds__(kFrBlock) __attribute__((amdgpu_waves_per_eu(2, 2))
 }
 
 // Workgroup (h, m) merges head h's nrec (at most 8) records into the row's state; thread t owns dims
-// 2 t, 2 t + 1. All: nrec is 8, known to the compiler, so that every address is at a fixed offset (three one-row
-// pages as a graph: 24.2 us, with the count as an argument 24.75).
+// 2 t, 2 t + 1. All: nrec is 8, known to the compiler, so that every load is at a fixed offset of a scalar address.
 template <bool All>
 __global__ __launch_bounds__(kFaBlock) void fattn_combine_kernel(const float* __restrict__ part, float* rmax,
                                                                  float* rsum, uint16_t* out, int first, int n) {
@@ -817,12 +818,12 @@ hipError_t launch_full_attention(const uint16_t* q, const uint16_t* k_pages, con
                                  const float* masks, int P, float* running_max, float* running_sum, uint16_t* out,
                                  int M, hipStream_t s, DevCtx* ctx) {
     const int nchunks = P * kFaChunks;
-    const bool many = M * P >= kFrMinRowPages;
     // One row, up to kFaSplitPages pages: one chunk per dim-split workgroup (P x 32 workgroups). More:
     // spans of chunks over all dims, at most kFaMaxRecords workgroups per row.
     const bool split = P <= kFaSplitPages;
     RowsSplit r = {0, split ? 1 : (nchunks + kFaMaxRecords - 1) / kFaMaxRecords, 1};
     r.nrec = (nchunks + r.tpw - 1) / r.tpw;
+    const bool many = M * P >= kFrMinRowPages && (split || M * r.nrec > ctx->cus);
     if (many) r = rows_split(M, nchunks, ctx->cus);
     else r.rows = kFattnRecords / r.nrec;
     for (int m0 = 0; m0 < M; m0 += r.rows) {

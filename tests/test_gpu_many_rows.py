@@ -64,7 +64,7 @@ def check_pages(d, got, label):
     gate(wo, go, f"{label} out")
 
 
-@pytest.mark.parametrize("P,M,kind", [(3, 7, "causal"), (3, 8, "causal"), (6, 13, "scattered"), (12, 2, "causal"),
+@pytest.mark.parametrize("P,M,kind", [(3, 7, "causal"), (3, 8, "causal"), (6, 13, "scattered"), (12, 2, "causal"), (10, 3, "causal"), (11, 3, "causal"),
                                       (2, 66, "empty"), (1, 24, "scattered")])
 def test_full_attention_rows(P, M, kind):
     need_gpu()
