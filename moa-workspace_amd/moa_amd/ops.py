@@ -72,13 +72,15 @@ _I32 = (torch.int32,)
 def _stream(t: torch.Tensor) -> int:
     """The current HIP stream of the current device (its handle as an int). The library serves a
     call from the scratch of the current device, so the call's tensors must live there: a tensor
-    of another device is refused here rather than run against the wrong device's scratch."""
+    of another device is refused here rather than run against the wrong device's scratch. The handle
+    is asked for as a number: torch.cuda.current_stream builds a Stream object around it, 1.14 us of
+    host time per call against 0.08, and the small calls are bound by the host."""
     dev = t.get_device()
     cur = torch.cuda.current_device()
     if dev != cur:
         raise ValueError(f"the call's tensors live on cuda:{dev} but the current device is cuda:{cur}; "
                          f"call it under torch.cuda.device({dev})")
-    return torch.cuda.current_stream(dev).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(dev)
 
 
 def _rows(x: torch.Tensor, width: int, name: str) -> int:
