@@ -505,7 +505,9 @@ __global__ __launch_bounds__(kFrBlock) __attribute__((amdgpu_waves_per_eu(2, 2))
         const int un = todo ? __builtin_ctzll(todo) : 0;
         __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's K rows are in LDS
         fr_barrier();                                          // and the others'; V's reads of the tile before are done
-        // per 16 slots four sums of 4 MFMAs, added in pairs: one long chain's rounding would show in running_sum;
+        // per 16 slots four sums of 4 MFMAs, sum c over dims 128 c .. + 127 and added up in that order, as in the
+        // one-row kernels: a row's scores, and its maximum, have the same bits in every kernel (running_sum is off
+        // by the rounding of the largest score, 1.5e-6 of it). Step n takes 32 dims of sum n % 4;
         // fragments four ahead of the MFMAs that use them; this tile's V beside them
         f32x4v sc[2][4];
         bf16x8 kf[2][4];
@@ -513,21 +515,22 @@ __global__ __launch_bounds__(kFrBlock) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int c = 0; c < 4; ++c) sc[i][c] = f32x4v{0.0f, 0.0f, 0.0f, 0.0f};
-        auto read_k = [&](int j) {
+        auto read_k = [&](int n) {
 #pragma unroll
             for (int i = 0; i < 2; ++i)
-                kf[i][j & 3] = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const uint8_t*>(ks) + (ka ^ (64 * (j & 3))) +
-                                                                (j >> 2) * 256 + i * 16 * 1024);
+                kf[i][n & 3] = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const uint8_t*>(ks) + (ka ^ (64 * (n >> 2))) +
+                                                                (n & 3) * 256 + i * 16 * 1024);
         };
 #pragma unroll
-        for (int j = 0; j < 4; ++j) read_k(j);
+        for (int n = 0; n < 4; ++n) read_k(n);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
+        for (int n = 0; n < 16; ++n) {
 #pragma unroll
             for (int i = 0; i < 2; ++i)
-                sc[i][j & 3] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[i][j & 3], as_bf16x8(qf[j]), sc[i][j & 3], 0, 0, 0);
-            if (j < 12) read_k(j + 4);
-            if (j & 1) issue(vrs, vs, u, j >> 1, (j >> 1) + 1);
+                sc[i][n & 3] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[i][n & 3], as_bf16x8(qf[4 * (n & 3) + (n >> 2)]),
+                                                                       sc[i][n & 3], 0, 0, 0);
+            if (n < 12) read_k(n + 4);
+            if (n & 1) issue(vrs, vs, u, n >> 1, (n >> 1) + 1);
             __builtin_amdgcn_sched_barrier(0);
         }
         // element (i, e): slot 32 sh + 16 i + 4 g + e
@@ -537,7 +540,7 @@ __global__ __launch_bounds__(kFrBlock) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                x[i][e] = (sc[i][0][e] + sc[i][1][e]) + (sc[i][2][e] + sc[i][3][e]);
+                x[i][e] = ((sc[i][0][e] + sc[i][1][e]) + sc[i][2][e]) + sc[i][3][e];
                 x[i][e] = (vb >> (16 * i + e) & 1) ? x[i][e] : -INFINITY;
                 mx = fmaxf(mx, x[i][e]);
             }

@@ -101,6 +101,22 @@ def test_one_page_call_of_many_rows():
     gate(few[2], many[2][:16], "pages: 19 rows and 16")
 
 
+@pytest.mark.parametrize("P,M", [(1, 17), (3, 6), (12, 3)])
+def test_running_max_has_the_same_bits_in_every_kernel(P, M):
+    """A score is summed in one order whichever kernel computes it: rows of a call that shares passes over
+    the pages, and each row by itself, page by page (one-row kernels) and over all pages."""
+    need_gpu()
+    from test_gpu_full import fused_gpu, pages_gpu
+    say(f"running max P={P} M={M}")
+    d = synth.cfg_full_attention(seed=7 * P + M, M=M, P=P, pos=P * TF - M - 3 + np.arange(M), q_std=1.0)
+    many = (fused_gpu(d), pages_gpu(d))
+    for m in range(M):
+        one = dict(d, q=np.ascontiguousarray(d["q"][m:m + 1]), masks=np.ascontiguousarray(d["masks"][:, m:m + 1]))
+        for got in (fused_gpu(one), pages_gpu(one)):
+            for w in many:
+                assert np.array_equal(w[0][m].reshape(-1), got[0].reshape(-1)), f"row {m}"
+
+
 @pytest.mark.parametrize("M,pos", [(17, 600), (65, 30)])
 def test_full_projection_rows(M, pos):
     need_gpu()
