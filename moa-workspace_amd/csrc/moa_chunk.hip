@@ -798,10 +798,12 @@ int pick_splits(int tiles, int ksteps, size_t rows_x_cols) {
 }
 
 // Weight rows per workgroup of a split-K projection: 64 where twice the tiles of 128-row tiles fill the device
-// with half the k splits, so half the f32 partial sums are written and read back: O up to 256 rows (at 256:
-// GEMM 17.3 -> 16.5 us, post rows 9.1 -> 6.9), QKV up to 128. Else 128, whose main loop does twice the MFMA
-// work per A load and per barrier, on eight waves: QKV of a 200-row full-attention layer (with O)
-// 72.6 -> 66.0 us, the 200-row FP8 layer 153 -> 150, 256 rows even; O at 1000 rows 484 -> 479 (layer). Down always
+// with half the k splits, so half the f32 partial sums are written and read back: the sliding layers' O (256 rows:
+// GEMM 17.3 -> 16.5 us, post rows 9.1 -> 6.9) and the full-attention O up to 256 rows, QKV up to 128. Else 128, whose
+// main loop does twice the MFMA work per A load and per barrier, on eight waves: QKV of a 200-row full-attention layer
+// (with O) 72.6 -> 66.0 us, the 200-row FP8 layer 153 -> 150, 256 rows even. (The sliding O of 1000 rows in 128-row
+// tiles gains 2 us of the layer's 487 but adds two halves of k, where 64 adds one chain: a sum's last bit flips a
+// few of its bf16 roundings, which the FFN carries on into 1 in 100 elements of the residual.) Down always
 // takes 128 (with 64, down measured 39.1 -> 44.6 us against 9.5 -> 7.1 us saved in its post rows), and so does the
 // full-attention QKV, whose 136 tiles of 64 rows would not split: with O, 20 rows 38.9 -> 37.1 us, 64 rows 44.8 ->
 // 40.2, 128 rows 52.5 -> 50.0 (the sliding QKV's 128 tiles do: 17..128 rows 0.3-1 us faster with 64).
@@ -919,7 +921,7 @@ static hipError_t o_chunk_gemm(const OParams& p, int m0, int M, hipStream_t s, D
     g.w[0] = p.ow; g.nseg[0] = 0; g.nseg[1] = kH; g.nsegs = 1;
     g.yf = ctx->fbuf;
     const int bm = pick_bm(M), mt = m_tiles(M, bm);
-    const bool narrow = M <= 256;
+    const bool narrow = !p.div || M <= 256;
     *sp = pick_splits(kH / (narrow ? kCkOBN : kCkBN) * mt, K / kCkBK, (size_t)M * kH);
     return narrow ? gemm_partial<FfnFormat::FP8, kCkOBN>(g, *sp, bm, s) : gemm_partial(g, *sp, bm, s);
 }

@@ -196,3 +196,27 @@ def test_ffn_row_tiles(fmt, M):
     want = getattr(F, "oracle_" + fmt)(dict(d, residual=d["residual"][rows].copy()))
     assert np.all(np.isfinite(unbf(got.reshape(-1))))
     gate(np.asarray(want).reshape(len(rows), -1), got[rows], f"ffn {fmt} M{M}", atol=F.FFN_ATOL)
+
+
+@pytest.mark.parametrize("M", [520, 769])
+def test_o_sums_of_long_chunks_run_in_one_chain(M):
+    """Past 512 rows the sliding O adds a column's 4096 products into one f32 chain, so a row's bits are those
+    that O has always given. The odd columns' sums stand midway between two bf16 values after the first product
+    ((1 + 2^-5)(1 + 2^-3), the lower of the two even); every later product is 2^-30, so the 16 that one matrix
+    instruction adds are under half an f32 step of that sum and leave it. Summed apart from it, as by a second k
+    split, 2048 of them are 2^-19 and push the rounding up. So the row with them and the row without must agree."""
+    need_gpu()
+    from test_gpu_o import run_gpu as o_gpu
+    say(f"o M={M}: sums in one chain")
+    d = synth.cfg_o(3, M=M)
+    x = np.zeros((M, 4096), np.float32)
+    x[:, 0] = 1.0 + 2.0 ** -5
+    x[1::2, 1:] = 2.0 ** -24
+    w = np.full((3840, 4096), 0x08, np.uint8)  # E4M3 2^-6
+    w[:, 0] = 0x38                              # 1
+    w[1::2, 0] = 0x39                           # 1.125
+    d.update(x=prng.f32_to_bf16_bits(x), o_weight=w, o_weight_scale=np.ones(3840, np.float32),
+             residual=np.zeros((M, 3840), np.uint16))
+    got = o_gpu(d)
+    assert not np.array_equal(got[0, 0::2], got[0, 1::2])
+    assert np.array_equal(got, np.broadcast_to(got[0], got.shape))
