@@ -663,7 +663,9 @@ __global__ __launch_bounds__(kCkBlock) void chunk_qkv_heads_kernel(QkvParams p, 
 // the partial sums: all loads of the RP rows, 16 bytes per lane, go out before any is used, and the
 // head's weights and scales are read once for them. 1000 rows
 // (33 MB of sums) 16 us, 256 rows (17 MB) 8; with a lane's four elements 64 apart in 4-byte loads, one row
-// per wave, 32 and 11.
+// per wave, 32 and 11. The squares of a head's 64-element quarters (16 lanes each) are added in the tree order of
+// ck_block_sum over chunk_qkv_heads_kernel's threads, distance 32 down to 1, then the quarters in turn: from equal
+// projections both kernels make equal bits.
 template <ScaleKind SK, int ZS, int RP>
 __global__ __launch_bounds__(kCkBlock) void chunk_qkv_head_rows_kernel(QkvParams p, int m0, int M,
                                                                        const float* __restrict__ part, uint32_t* err) {
@@ -710,13 +712,19 @@ __global__ __launch_bounds__(kCkBlock) void chunk_qkv_head_rows_kernel(QkvParams
             a[2] += pz[i][z].z;
             a[3] += pz[i][z].w;
         }
-        float ss = 0.0f;
+        float ss[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             a[e] = rbf(a[e] * sc[e]);
-            ss = fmaf(a[e], a[e], ss);
+            ss[e] = a[e] * a[e];
+#pragma unroll
+            for (int x = 8; x >= 1; x >>= 1) ss[e] += __shfl_xor(ss[e], x);
         }
-        const float inv = rms_inverse(wave_sum(ss), kDs);
+        const uint32_t quarter = __float_as_uint((ss[0] + ss[2]) + (ss[1] + ss[3]));
+        float tot = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) tot += __uint_as_float(__builtin_amdgcn_readlane(quarter, 16 * k));
+        const float inv = rms_inverse(tot, kDs);
         float n[4], o[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {

@@ -220,3 +220,27 @@ def test_o_sums_of_long_chunks_run_in_one_chain(M):
     got = o_gpu(d)
     assert not np.array_equal(got[0, 0::2], got[0, 1::2])
     assert np.array_equal(got, np.broadcast_to(got[0], got.shape))
+
+
+def test_qkv_heads_bits_in_every_call_size():
+    """Rows with one non-zero input have projections of one product, the same in any order of summation; the head
+    norms' sums of squares are added in one order too, so a 300-row call and 16-row calls agree in every bit."""
+    need_gpu()
+    from test_gpu_qkv import run_gpu as qkv_gpu
+    say("qkv: 300 rows and 16 at a time")
+    M, pos = 300, 40
+    d = synth.cfg_qkv(5, M=M, pos=pos)
+    x = np.zeros((M, 3840), np.float32)
+    x[np.arange(M), 11 * np.arange(M)] = 1.0 + np.arange(M) / 512.0
+    d["x"] = prng.f32_to_bf16_bits(x)
+    q, k, v = qkv_gpu(d, M)
+    q = np.asarray(q).reshape(M, -1)
+    for m in range(0, M, 16):
+        n = min(16, M - m)
+        few = dict(d, x=np.ascontiguousarray(d["x"][m:m + n]), rope_offset=(pos + m) * 256 * 2,
+                   kv_offset=(pos + m) * 8 * 256 * 2)
+        qf, kf, vf = qkv_gpu(few, n)
+        at = slice(pos + m, pos + m + n)
+        assert np.array_equal(q[m:m + n], np.asarray(qf).reshape(n, -1)), f"q of rows {m} .."
+        assert np.array_equal(np.asarray(k)[at], np.asarray(kf)[at]), f"k of rows {m} .."
+        assert np.array_equal(np.asarray(v)[at], np.asarray(vf)[at]), f"v of rows {m} .."
