@@ -228,13 +228,14 @@ __global__ __launch_bounds__(kAtBlock) void attn_split_kernel(const uint16_t* __
 // with an online softmax of its own, on v_mfma_f32_32x32x16_bf16, transposed: scores^T = K Q^T and
 // out^T += V^T P^T, so that a lane holds one query row's values. The weights stay in the registers
 // they are computed in -- step kk of the second product takes slots 16 kk + 4 h + {0..3, 8..11} from
-// lane half h, for V (transposing LDS reads) alike -- and enter as two bf16 parts, high and low (about
-// 16 significant bits; sums of weights are f32 of the whole weights). K and V tiles are loaded a tile
-// ahead into registers, in whole rows, and pass through the wave's own LDS: no barrier in the loop.
+// lane half h, for V (transposing LDS reads) alike -- and enter as three bf16 parts, which hold the 24 bits
+// of the f32 weight that attn_split_kernel multiplies by (two parts: 16-17 bits, 1-2 us less at 512 rows). K and V
+// tiles are loaded a tile ahead into registers, in whole rows, and pass through the wave's own LDS: no barrier in
+// the loop.
 // The waves' states meet in LDS at the end; with several parts (few rows: the slots are spread over
 // up to 8 workgroups), the parts' in attn_merge_kernel.
 // Bound: a workgroup reads every valid slot's K and V of its head once (1 MB of 1024 slots) through the
-// CU's L1, as long as the 48 MFMAs per tile and wave take. 512 rows
+// CU's L1, as long as the 64 MFMAs per tile and wave take. 512 rows
 // (causal, from position 300) 30 us, over all slots 34; 1000 rows 57; 16 rows 12 (a workgroup set per row,
 // as above: 693, 694, 1357, 22).
 constexpr int kArRows = 16;                     // token rows per workgroup
@@ -402,14 +403,16 @@ __global__ __launch_bounds__(kAtBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
         }
         const float mu = m_ref == -INFINITY ? 0.0f : m_ref;
         float ls = 0.0f;
-        uint32_t ph[8], pl[8];
+        uint32_t ph[8], pm[8], pl[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const float p0 = __expf(sc[0][2 * i] - mu), p1 = __expf(sc[0][2 * i + 1] - mu);
             ls += p0;
             ls += p1;
             ph[i] = pk_bf16(p0, p1);
-            pl[i] = pk_bf16(p0 - __uint_as_float(ph[i] << 16), p1 - __uint_as_float(ph[i] & 0xffff0000u));
+            const float r0 = p0 - __uint_as_float(ph[i] << 16), r1 = p1 - __uint_as_float(ph[i] & 0xffff0000u);
+            pm[i] = pk_bf16(r0, r1);
+            pl[i] = pk_bf16(r0 - __uint_as_float(pm[i] << 16), r1 - __uint_as_float(pm[i] & 0xffff0000u));
         }
         l_run = fmaf(l_run, scale, ls + __shfl_xor(ls, 32));
         if (__any(scale != 1.0f)) {
@@ -435,10 +438,13 @@ __global__ __launch_bounds__(kAtBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
             if (x < 14) read_v(vf[(x + 2) % 3], x + 2);
             load_v(vo, x);
             const int k = 4 * (x >> 3);
-            o[x & 7] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                vf[x % 3], __builtin_bit_cast(bf16x8, make_uint4(ph[k], ph[k + 1], ph[k + 2], ph[k + 3])), o[x & 7], 0, 0, 0);
-            o[x & 7] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                vf[x % 3], __builtin_bit_cast(bf16x8, make_uint4(pl[k], pl[k + 1], pl[k + 2], pl[k + 3])), o[x & 7], 0, 0, 0);
+            auto add = [&](const uint32_t (&w)[8]) {
+                o[x & 7] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    vf[x % 3], __builtin_bit_cast(bf16x8, make_uint4(w[k], w[k + 1], w[k + 2], w[k + 3])), o[x & 7], 0, 0, 0);
+            };
+            add(ph);
+            add(pm);
+            add(pl);
             __builtin_amdgcn_sched_barrier(0);
         }
         u = un;

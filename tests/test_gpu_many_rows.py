@@ -244,3 +244,33 @@ def test_qkv_heads_bits_in_every_call_size():
         assert np.array_equal(q[m:m + n], np.asarray(qf).reshape(n, -1)), f"q of rows {m} .."
         assert np.array_equal(np.asarray(k)[at], np.asarray(kf)[at]), f"k of rows {m} .."
         assert np.array_equal(np.asarray(v)[at], np.asarray(vf)[at]), f"v of rows {m} .."
+
+
+@pytest.mark.parametrize("M", [3, 6, 130])
+def test_sliding_attention_weights_keep_their_f32_bits(M):
+    """Three slots with scores 0, 0 and -s: out = (p - hi - lo) / (2 + p) with p = exp(-s) on a value of 1 and
+    hi, lo, the bf16 parts of p nearest first, as the other slots' values with their signs turned. Only bits of
+    p below its first 16 are left. Bound: the largest f32 step of |s log2 e| < 1 and of exp2's result is 2^-24,
+    two of each and three sums of as much below 1 stay under 2^-21 in the numerator (2^-18 here); bf16 output."""
+    need_gpu()
+    from test_gpu_attention import run_gpu
+    say(f"attention M={M}: bits of the weights")
+    s = 77.0 / 128.0
+    bf = lambda x: float(unbf(prng.f32_to_bf16_bits(np.array([x], np.float32)))[0])
+    p = float(np.exp(np.float64(-s)))
+    hi = bf(p)
+    lo = bf(p - hi)
+    d = synth.cfg_attention(seed=M, M=M)
+    k = np.zeros((TS, 8, 256), np.float32)
+    v = np.zeros((TS, 8, 256), np.float32)
+    q = np.zeros((M, 8, 2, 256), np.float32)
+    q[..., 0] = 1.0
+    k[9, :, 0] = -s
+    v[5], v[9], v[20] = -hi, 1.0, -lo
+    mask = np.zeros((M, TS), np.float32)
+    mask[:, [5, 9, 20]] = 1.0
+    d.update(q=prng.f32_to_bf16_bits(q), k_cache=prng.f32_to_bf16_bits(k), v_cache=prng.f32_to_bf16_bits(v), mask=mask)
+    got = unbf(run_gpu(d).reshape(-1)).astype(np.float64)
+    want = (p - hi - lo) / (2.0 + p)
+    assert abs(want) > 2.0 ** -20
+    assert np.all(np.abs(got - want) <= 2.0 ** -21 / (2.0 + p) + 2.0 ** -8 * abs(want)), (got.min(), got.max(), want)
