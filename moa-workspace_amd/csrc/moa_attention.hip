@@ -224,10 +224,12 @@ __global__ __launch_bounds__(kAtBlock) void attn_split_kernel(const uint16_t* __
 
 // ---------------------------------------------------------------- many token rows
 // Workgroup (n, y, z): head n, token rows 16 y .. + 15 with both query heads (32 query rows), part z of
-// the slots. The four waves take 32-slot tiles in turn (those in which some row has a valid slot), each
-// with an online softmax of its own, on v_mfma_f32_32x32x16_bf16, transposed: scores^T = K Q^T and
-// out^T += V^T P^T, so that a lane holds one query row's values. The weights stay in the registers
-// they are computed in -- step kk of the second product takes slots 16 kk + 4 h + {0..3, 8..11} from
+// the slots. The four waves take the 32-slot tiles in which some row has a valid slot, dealt by the tile's number,
+// so that a row's sums run in one order whichever rows stand beside it: wave w one tile of every four, turned by one
+// from four to four, so that masks with a period of 2 or 4 tiles keep all waves busy (tiles w, w + 4, ..: 31.1 us for
+// 20.2 with every other tile valid, 512 rows). Each has an online softmax of its own, on
+// v_mfma_f32_32x32x16_bf16, transposed: scores^T = K Q^T and out^T += V^T P^T, so that a lane holds one query
+// row's values. The weights stay in the registers they are computed in -- step kk of the second product takes slots 16 kk + 4 h + {0..3, 8..11} from
 // lane half h, for V (transposing LDS reads) alike -- and enter as three bf16 parts, which hold the 24 bits
 // of the f32 weight that attn_split_kernel multiplies by (two parts: 16-17 bits, 1-2 us less at 512 rows). K and V
 // tiles are loaded a tile ahead into registers, in whole rows, and pass through the wave's own LDS: no barrier in
@@ -236,7 +238,7 @@ __global__ __launch_bounds__(kAtBlock) void attn_split_kernel(const uint16_t* __
 // up to 8 workgroups), the parts' in attn_merge_kernel.
 // Bound: a workgroup reads every valid slot's K and V of its head once (1 MB of 1024 slots) through the
 // CU's L1, as long as the 64 MFMAs per tile and wave take. 512 rows
-// (causal, from position 300) 30 us, over all slots 34; 1000 rows 57; 16 rows 12 (a workgroup set per row,
+// (causal, from position 300) 29 us, over all slots 33; 1000 rows 56; 16 rows 12 (a workgroup set per row,
 // as above: 693, 694, 1357, 22).
 constexpr int kArRows = 16;                     // token rows per workgroup
 constexpr int kArQ = kArRows * kGs;             // query rows
@@ -330,12 +332,10 @@ __global__ __launch_bounds__(kAtBlock) __attribute__((amdgpu_waves_per_eu(1, 1))
     uint32_t mine = 0;  // this wave's tiles
     {
         uint32_t any = 0;
-        if (lane < nt)
+        if (lane < nt && ((lane + (lane >> 2)) & 3) == wave)
 #pragma unroll
             for (int r = 0; r < kArRows; ++r) any |= (uint32_t)(bits[r][(u0 + lane) / 2] >> (32 * ((u0 + lane) & 1)));
-        uint32_t todo = (uint32_t)__ballot(any != 0);
-        for (int c = 0; todo; ++c, todo &= todo - 1)
-            if ((c & 3) == wave) mine |= todo & -todo;
+        mine = (uint32_t)__ballot(any != 0);
     }
 
     // LDS addresses: writes (row 2 i + hf: i % 8 here, i / 8 as 16 rows), K reads (chunk 2 j + hf of row l32:

@@ -274,3 +274,22 @@ def test_sliding_attention_weights_keep_their_f32_bits(M):
     want = (p - hi - lo) / (2.0 + p)
     assert abs(want) > 2.0 ** -20
     assert np.all(np.abs(got - want) <= 2.0 ** -21 / (2.0 + p) + 2.0 ** -8 * abs(want)), (got.min(), got.max(), want)
+
+
+@pytest.mark.parametrize("M", [130, 260])
+def test_sliding_attention_row_does_not_depend_on_its_neighbours(M):
+    """A row with valid slots in every other 32-slot tile keeps its bits whichever tiles the other rows of the
+    call need."""
+    need_gpu()
+    from test_gpu_attention import run_gpu
+    say(f"attention M={M}: a row beside others")
+    d = synth.cfg_attention(seed=M, M=M, q_std=0.1)
+    sparse = (np.arange(TS) // 32 % 2 == 0).astype(np.float32)
+    d["mask"] = np.broadcast_to(sparse, (M, TS)).copy()
+    alone = run_gpu(d)
+    d["mask"] = np.ones((M, TS), np.float32)
+    rows = [0, 21, M - 1]
+    d["mask"][rows] = sparse
+    beside = run_gpu(d)
+    for m in rows:
+        assert np.array_equal(alone[m], beside[m]), f"row {m}"
