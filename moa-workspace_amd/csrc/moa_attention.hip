@@ -229,11 +229,11 @@ __global__ __launch_bounds__(kAtBlock) void attn_split_kernel(const uint16_t* __
 // from four to four, so that masks with a period of 2 or 4 tiles keep all waves busy (tiles w, w + 4, ..: 31.1 us for
 // 20.2 with every other tile valid, 512 rows). Each has an online softmax of its own, on
 // v_mfma_f32_32x32x16_bf16, transposed: scores^T = K Q^T and out^T += V^T P^T, so that a lane holds one query
-// row's values. The weights stay in the registers they are computed in -- step kk of the second product takes slots 16 kk + 4 h + {0..3, 8..11} from
-// lane half h, for V (transposing LDS reads) alike -- and enter as three bf16 parts, which hold the 24 bits
-// of the f32 weight that attn_split_kernel multiplies by (two parts: 16-17 bits, 1-2 us less at 512 rows). K and V
-// tiles are loaded a tile ahead into registers, in whole rows, and pass through the wave's own LDS: no barrier in
-// the loop.
+// row's values. The weights stay in the registers they are computed in -- step kk of the second product takes slots
+// 16 kk + 4 h + {0..3, 8..11} from lane half h, for V (transposing LDS reads) alike -- and enter as three bf16 parts,
+// which hold the 24 bits of the f32 weight that attn_split_kernel multiplies by (two parts: 16-17 bits, 1-2 us less at
+// 512 rows). K and V tiles are loaded a tile ahead into registers, in whole rows, and pass through the wave's own LDS:
+// no barrier in the loop.
 // The waves' states meet in LDS at the end; with several parts (few rows: the slots are spread over
 // up to 8 workgroups), the parts' in attn_merge_kernel.
 // Bound: a workgroup reads every valid slot's K and V of its head once (1 MB of 1024 slots) through the
@@ -553,15 +553,10 @@ hipError_t launch_sliding_attention(const uint16_t* q, const uint16_t* k_cache, 
         hipLaunchKernelGGL(attn_merge_kernel, dim3(kNs, M), dim3(kAtBlock), 0, s, (const float*)ctx->attn_part, nz, out);
         return hipGetLastError();
     }
-    for (int m0 = 0; m0 < M; m0 += kMaxDecodeM) {
-        const int mm = M - m0 < kMaxDecodeM ? M - m0 : kMaxDecodeM;
-        hipLaunchKernelGGL(attn_split_kernel, dim3(kNs, kAtChunks, mm), dim3(kAtBlock), 0, s,
-                           q + (size_t)m0 * kQs, k_cache, v_cache, mask + (size_t)m0 * kTs, out + (size_t)m0 * kQs,
-                           ctx->attn_part, ctx->tickets + kTicketAttn * kTicketStride);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
+    static_assert(kArMinRows <= kMaxDecodeM + 1, "one launch's partials and tickets");
+    hipLaunchKernelGGL(attn_split_kernel, dim3(kNs, kAtChunks, M), dim3(kAtBlock), 0, s, q, k_cache, v_cache, mask, out,
+                       ctx->attn_part, ctx->tickets + kTicketAttn * kTicketStride);
+    return hipGetLastError();
 }
 
 }  // namespace moa

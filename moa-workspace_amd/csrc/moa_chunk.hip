@@ -129,9 +129,9 @@ constexpr int kCkNt = 0;
 //   permutation of the step's 64 k. Row blocks past M read zeros (the buffer ends there); rows
 //   past M are not stored.
 //   Weights (FP8) are staged once per workgroup through LDS, widened to bf16 on the way (exact for
-//   E4M3; once per workgroup instead of once per wave): each thread moves one 16-byte chunk (with four waves
-//   two) per step, loaded eight steps ahead (HBM latency at the rate the whole chip streams weights) and
-//   written two steps ahead; a wave reads 64 bytes (bf16) per lane per 32-column block.
+//   E4M3; once per workgroup instead of once per wave): each thread moves one 16-byte chunk per step, loaded
+//   eight steps ahead (HBM latency at the rate the whole chip streams weights) and written two steps ahead;
+//   a wave reads 64 bytes (bf16) per lane per 32-column block.
 //   All loads are buffer loads whose per-lane offsets are fixed: the step moves the scalar
 //   offset only. Prefetches past the last step repeat the last step (harmless), so the loop body
 //   has no branches.
@@ -153,7 +153,7 @@ void chunk_gemm_kernel(GemmArgs g) {
     constexpr int KG = BN == 128 && BM == 64 ? 2 : 1, CG = NW / RG / KG, JN = 4 / KG;  // JN: MFMAs per block and step
     static_assert(BM == 256 || BM == 128 || BM == 64, "row tiles");
     constexpr int NB = BN / 32 / CG;   // 32-column blocks per wave
-    constexpr int RPT = BN / (16 * NW);  // staged weight rows per thread
+    static_assert(BN == 16 * NW, "a thread stages 16 bytes of one weight row per step");
     constexpr bool FP4 = F != FfnFormat::FP8;
     // bytes per weight row and per 64-k step; FP4 block-scale bytes per row and per step
     const int rb = FP4 ? g.K / 2 : g.K;
@@ -172,40 +172,33 @@ void chunk_gemm_kernel(GemmArgs g) {
     const int m_wave = m_blk + rg * 32 * MB;
     const int kz = g.K / gridDim.z, kbeg = blockIdx.z * kz, nsteps = kz / kCkBK;
 
-    // staged weight rows of this thread: tile row r0 (and, four waves on BN = 128, r0 + 64), k 16 q .. 16 q + 15 of each step
-    // (FP8: 16 bytes; FP4: 8 bytes of codes and the one block-scale code covering them)
+    // staged weights of this thread: tile row r0, k 16 q .. 16 q + 15 of each step (FP8: 16 bytes; FP4: 8 bytes of codes
+    // and the one block-scale code covering them)
     const int r0 = t >> 2, q = t & 3;
-    __amdgpu_buffer_rsrc_t wrs[2], srs[2];
-    int wvo[2], svo[2] = {0, 0};
+    __amdgpu_buffer_rsrc_t wrs, srs;
+    int wvo, svo = 0;
     const int kcol = FP4 ? (kbeg + 16 * q) / 2 : kbeg + 16 * q;
     const int scol = F == FfnFormat::NVFP4 ? kbeg / 16 + q : kbeg / 32 + q / 2;
     int seg = 0;
     if constexpr (E == Epi::GeGLU) {
-        const size_t off = (size_t)blockIdx.x * 64 * rb;
-        wrs[0] = ck_rsrc(g.w[0] + off, 64u * rb);
-        wrs[1] = ck_rsrc(g.w2 + off, 64u * rb);
-        if (NW == 8 && __builtin_amdgcn_readfirstlane(wave) >= 4) wrs[0] = wrs[1];  // waves 4 .. 7 stage the gate rows
-        wvo[0] = wvo[1] = (r0 & 63) * rb + kcol;
+        const bool gate = __builtin_amdgcn_readfirstlane(wave) >= 4;  // waves 0 .. 3 stage the up rows, 4 .. 7 the gate rows
+        wrs = ck_rsrc((gate ? g.w2 : g.w[0]) + (size_t)blockIdx.x * 64 * rb, 64u * rb);
+        wvo = (r0 & 63) * rb + kcol;
         if constexpr (FP4) {
-            const size_t so = (size_t)blockIdx.x * 64 * sb;
-            srs[0] = ck_rsrc(g.wsc[0] + so, 64u * sb);
-            srs[1] = ck_rsrc(g.wsc2 + so, 64u * sb);
-            if (NW == 8 && __builtin_amdgcn_readfirstlane(wave) >= 4) srs[0] = srs[1];
-            svo[0] = svo[1] = (r0 & 63) * sb + scol;
+            srs = ck_rsrc((gate ? g.wsc2 : g.wsc[0]) + (size_t)blockIdx.x * 64 * sb, 64u * sb);
+            svo = (r0 & 63) * sb + scol;
         }
     } else {
         const int n0 = blockIdx.x * BN;
         while (seg + 1 < g.nsegs && n0 >= g.nseg[seg + 1]) ++seg;
-        wrs[0] = wrs[1] = ck_rsrc(g.w[seg] + (size_t)(n0 - g.nseg[seg]) * rb, (uint32_t)BN * rb);
-        wvo[0] = r0 * rb + kcol;
-        wvo[1] = (r0 + 64) * rb + kcol;
+        wrs = ck_rsrc(g.w[seg] + (size_t)(n0 - g.nseg[seg]) * rb, (uint32_t)BN * rb);
+        wvo = r0 * rb + kcol;
         if constexpr (FP4) {
-            srs[0] = srs[1] = ck_rsrc(g.wsc[seg] + (size_t)(n0 - g.nseg[seg]) * sb, (uint32_t)BN * sb);
-            svo[0] = r0 * sb + scol;
-            svo[1] = (r0 + 64) * sb + scol;
+            srs = ck_rsrc(g.wsc[seg] + (size_t)(n0 - g.nseg[seg]) * sb, (uint32_t)BN * sb);
+            svo = r0 * sb + scol;
         }
     }
-    const int wdst0 = r0 * kCkWStride + 32 * q, wdst1 = (r0 + 64) * kCkWStride + 32 * q;
+    const int wdst = r0 * kCkWStride + 32 * q;
 
     const int kst = g.K / kCkBK;  // 64-k steps (A tiles) per row block
     const int rblks = (min(g.M - m_blk, BM) + 31) >> 5;
@@ -223,38 +216,30 @@ void chunk_gemm_kernel(GemmArgs g) {
             for (int r = 0; r < 16; ++r) acc[mb][nb][r] = 0.0f;
 
     constexpr int WD = 6;  // weight register sets: W(s + 2) is loaded six steps before it is staged
-    uint4 wr[WD][2];       // [set][row pair]
+    uint4 wr[WD];          // [set]
     uint4 ar[3][MB][JN];   // [set][32-row block][16 bytes]: A(s) in set s mod 3, loaded two steps ahead
     bf16x8 bb[2][JN];      // B fragments: [set][MFMA j]
     const int last = nsteps - 1;
     // FP4: .x, .y the 16 codes, .z the block-scale code
-    auto load_w = [&](uint4 (&dst)[2], int s) {
+    auto load_w = [&](uint4& dst, int s) {
         const int so = min(s, last) * kStepB;
         if constexpr (FP4) {
-#pragma unroll
-            for (int i = 0; i < RPT; ++i) {
-                const auto v = __builtin_amdgcn_raw_buffer_load_b64(wrs[i], wvo[i], so, kCkNt);
-                dst[i].x = v[0];
-                dst[i].y = v[1];
-                dst[i].z = __builtin_amdgcn_raw_buffer_load_b8(srs[i], svo[i], min(s, last) * kStepS, 0);
-            }
+            const auto v = __builtin_amdgcn_raw_buffer_load_b64(wrs, wvo, so, kCkNt);
+            dst.x = v[0];
+            dst.y = v[1];
+            dst.z = __builtin_amdgcn_raw_buffer_load_b8(srs, svo, min(s, last) * kStepS, 0);
         } else {
-#pragma unroll
-            for (int i = 0; i < RPT; ++i)
-                dst[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wrs[i], wvo[i], so, kCkNt));
+            dst = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wrs, wvo, so, kCkNt));
         }
     };
-    auto store_w = [&](const uint4 (&src)[2], int buf) {
-#pragma unroll
-        for (int i = 0; i < RPT; ++i) {
-            bf16x8* d = reinterpret_cast<bf16x8*>(&ws[buf][i ? wdst1 : wdst0]);
-            if constexpr (FP4) {
-                d[0] = fp4x8_to_bf16<F>(src[i].x, src[i].z);
-                d[1] = fp4x8_to_bf16<F>(src[i].y, src[i].z);
-            } else {
-                d[0] = fp8x8_to_bf16(src[i].x, src[i].y);
-                d[1] = fp8x8_to_bf16(src[i].z, src[i].w);
-            }
+    auto store_w = [&](const uint4& src, int buf) {
+        bf16x8* d = reinterpret_cast<bf16x8*>(&ws[buf][wdst]);
+        if constexpr (FP4) {
+            d[0] = fp4x8_to_bf16<F>(src.x, src.z);
+            d[1] = fp4x8_to_bf16<F>(src.y, src.z);
+        } else {
+            d[0] = fp8x8_to_bf16(src.x, src.y);
+            d[1] = fp8x8_to_bf16(src.z, src.w);
         }
     };
     auto load_a = [&](uint4 (&dst)[MB][JN], int s) {
@@ -282,7 +267,7 @@ void chunk_gemm_kernel(GemmArgs g) {
     // Three LDS buffers: step s reads buffer s mod 3 and stages W(s + 2) into buffer (s + 2) mod 3
     // (last read in step s - 1, before the barrier that opens step s), so the first fragment of
     // step s + 1 (buffer (s + 1) mod 3, staged in step s - 1) is read before step s ends. Within a
-    // step, fragment nb + 1 is read while fragment nb's eight MFMAs run.
+    // step, fragment nb + 1 is read while fragment nb's JN MB MFMAs run.
 #pragma unroll
     for (int i = 0; i < WD; ++i) load_w(wr[i], i);
     load_a(ar[0], 0);
@@ -368,8 +353,8 @@ void chunk_gemm_kernel(GemmArgs g) {
         constexpr int cb = c % 3, nbuf = (c + 1) % 3;
         const uint4(&a)[MB][JN] = ar[c % 3];
         constexpr int kDsR = 0x100, kDsW = 0x200, kVmR = 0x020, kValu = 0x002, kMfma = 0x008;
-        constexpr int kWLoads = (FP4 ? 2 : 1) * RPT * (BN == 64 ? 1 : c & 1 ? 2 : 0);
-        constexpr int kWValu = (F == FfnFormat::NVFP4 ? 4 : 1) * RPT * 8 / kMf;
+        constexpr int kWLoads = (FP4 ? 2 : 1) * (BN == 64 ? 1 : c & 1 ? 2 : 0);
+        constexpr int kWValu = (F == FfnFormat::NVFP4 ? 4 : 1) * 8 / kMf;
         read_b(bb[1], cb, 1);
         store_w(wr[(c + 2) % WD], (c + 2) % 3);
         mfma8(a, bb[0], Par<0>{});
@@ -473,7 +458,7 @@ void chunk_gemm_kernel(GemmArgs g) {
     }
     if (m_wave >= g.M) return;
     // Accumulator element r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4 of the 32-row block,
-    // column l % 32 of the 32-column block. A wave whose 64 rows all lie below M stores without
+    // column l % 32 of the 32-column block. A wave whose 32 MB rows all lie below M stores without
     // per-element tests (a test per element would serialise the 64-128 element computations).
     const bool full = m_wave + 32 * MB <= g.M;
     if constexpr (E == Epi::F32Partial) {
@@ -488,8 +473,8 @@ void chunk_gemm_kernel(GemmArgs g) {
                     if (full || m < g.M) yz[(size_t)m * g.N + CG * nb * 32] = acc[mb][nb][r];
                 }
     } else {
-        // p = bf16(gelu(gate) * up) for the wave's 64 rows x 64 columns, transposed through the
-        // wave's own 9 KB of LDS (row stride 72 elements) so that each lane then stores whole
+        // p = bf16(gelu(gate) * up) for the wave's 32 MB rows x 64 / CG columns, transposed through the
+        // wave's own LDS (row stride 72 elements) so that each lane then stores whole
         // 16-byte units of the A tiles (row, 8 consecutive columns).
         uint16_t* tp = reinterpret_cast<uint16_t*>(smem + kRedBytes) + (rg * CG + cg) * (32 * MB * kTpStride);
         // the format's commit of each projection: FP8 bf16(sum * s[n]); NVFP4 bf16(bf16(sum) * 1/g);
