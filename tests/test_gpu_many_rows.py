@@ -293,3 +293,169 @@ def test_sliding_attention_row_does_not_depend_on_its_neighbours(M):
     beside = run_gpu(d)
     for m in rows:
         assert np.array_equal(alone[m], beside[m]), f"row {m}"
+
+
+def long_pages(P, M, kind):
+    """Pages whose scores grow from tile to tile, so that a row's reference moves several times over a workgroup's
+    tiles. scattered: random masks, tile 5 of every page and all of page 1 nobody's, a row with one late slot and a
+    row with none."""
+    rng = np.random.default_rng(1000 * P + M)
+    grow = np.linspace(0.3, 1.0, P * 8, dtype=np.float32).reshape(P, 8, 1, 1)
+    k = rng.standard_normal((P, 8, 64, 512), np.float32) * grow
+    masks = synth.full_masks(P, P * TF - M - 100 + np.arange(M))
+    if kind == "scattered":
+        masks = (rng.random((P, M, TF), np.float32) < 0.3).astype(np.float32)
+        masks[:, :, 320:384] = 0.0
+        masks[1] = 0.0
+        masks[:, M // 2] = 0.0
+        masks[P - 1, M // 2, 500] = 1.0
+        masks[:, M - 2] = 0.0
+    b = prng.f32_to_bf16_bits
+    return dict(q=b(rng.standard_normal((M, 16, 512), np.float32)), k_pages=b(k.reshape(P, TF, 512)),
+                v_pages=b(rng.standard_normal((P, TF, 512), np.float32)), masks=masks)
+
+
+@pytest.mark.parametrize("P,M,kind", [(6, 200, "causal"), (6, 200, "scattered"), (20, 40, "scattered"), (40, 130, "causal"),
+                                      (64, 130, "scattered")])
+def test_full_attention_rows_over_many_tiles(P, M, kind):
+    """On 256 CUs 10, 7, 46 and 64 tiles per workgroup (200, 40, 130 and 130 rows): the pipeline beyond its first
+    tiles, tiles left out between others, repeated rescaling and every pass over the mask bits. 130 rows of 64 pages
+    are two launches, of 128 rows and of 2."""
+    need_gpu()
+    from test_gpu_full import fused_gpu
+    say(f"full attention P={P} M={M} {kind}")
+    d = long_pages(P, M, kind)
+    got = fused_gpu(d)
+    rows = sorted({0, 3, 4, M // 2, min(127, M - 3), M - 2, M - 1})
+    few = dict(d, q=np.ascontiguousarray(d["q"][rows]), masks=np.ascontiguousarray(d["masks"][:, rows]))
+    check_pages(few, [x[rows] for x in got], f"pages P{P} M{M} {kind}")
+    if kind == "scattered":
+        assert np.all(got[0][M - 2] == -np.inf) and not got[1][M - 2].any() and not got[2][M - 2].any()
+        assert np.all(got[1][M // 2] == 1.0)
+        assert np.array_equal(got[2][M // 2].reshape(16, 512), np.broadcast_to(d["v_pages"][P - 1, 500], (16, 512)))
+
+
+@pytest.mark.parametrize("M", [129, 256, 257, 300])
+def test_full_projection_row_tiles(M):
+    """The 256-row tile in one and two row blocks, QKV with two splits and one, O on 64 and 128 weight rows, and the
+    division by the sums over XCD-ordered rows."""
+    need_gpu()
+    from moa_amd import ops
+    from test_gpu_full import out_gpu, out_oracle, qkv_gpu, qkv_oracle
+    say(f"full qkv and output M={M}")
+    pos, rows = 5, sorted({0, 31, 63, 64, 127, 128, min(256, M - 1), M - 1})
+    d = synth.cfg_full_qkv(seed=M, M=M, pos=pos)
+    gq, gk, gv = qkv_gpu(d, M)
+    assert ops.device_errors() == 0
+    for m in rows:
+        one = dict(d, x=d["x"][m:m + 1], rope_offset=(pos + m) * 1024, kv_offset=(pos + m) * 1024)
+        wq, wk, wv = qkv_oracle(one, 1)
+        gate_rope(wq, gq[m:m + 1], f"full q_out M{M} row {m}", 512)
+        gate_rope(wk[pos + m], gk[pos + m], f"full k M{M} row {m}", 512)
+        gate(wv[pos + m], gv[pos + m], f"full v M{M} row {m}")
+    keep = np.setdiff1d(np.arange(TF), pos + np.arange(M))
+    assert np.array_equal(gk[keep], d["k_cache"][keep]) and np.array_equal(gv[keep], d["v_cache"][keep])
+    o = synth.cfg_full_o(seed=M, M=M)
+    o["running_sum"][M - 1, 0] = 0.0  # heads with no valid slot
+    o["running_sum"][64, 15] = 0.0
+    few = dict(o, x=o["x"][rows].copy(), running_sum=o["running_sum"][rows].copy(), residual=o["residual"][rows].copy())
+    gate(out_oracle(few), out_gpu(o)[rows], f"full output M{M}")
+
+
+def test_full_output_call_of_two_chunks():
+    """1030 rows are a chunk of 1024 and one of 6: the first chunk's bits are those of a 1024-row call, and the last
+    rows use their own sums."""
+    need_gpu()
+    from test_gpu_full import out_gpu, out_oracle
+    say("full output: 1030 rows")
+    o = synth.cfg_full_o(seed=30, M=1030)
+    o["running_sum"][1027, 2] = 0.0
+    part = lambda lo, hi: dict(o, **{k: np.ascontiguousarray(o[k][lo:hi]) for k in ("x", "running_sum", "residual")})
+    got = out_gpu(o)
+    assert np.array_equal(got[:1024], out_gpu(part(0, 1024)))
+    gate(out_oracle(part(1024, 1030)), got[1024:], "full output, rows 1024 .. 1029")
+
+
+def test_full_qkv_call_of_two_chunks_past_the_page():
+    """520 rows from slot 0 are a chunk of 512 and one of 8, whose rows fall past the page: the page and q_out of
+    the first 512 are those of a 512-row call, and the others write nothing and are reported."""
+    need_gpu()
+    from moa_amd import _lib, ops
+    from test_gpu_full import qkv_gpu
+    say("full qkv: 520 rows")
+    d = synth.cfg_full_qkv(seed=52, M=520, pos=0)
+    gq, gk, gv = qkv_gpu(d, 520)
+    assert ops.device_errors() == _lib.DEVERR_KV_OFFSET
+    hq, hk, hv = qkv_gpu(dict(d, x=np.ascontiguousarray(d["x"][:512])), 512)
+    assert ops.device_errors() == 0
+    assert np.array_equal(gq[:512], hq) and np.array_equal(gk, hk) and np.array_equal(gv, hv)
+    assert not gq[512:].any()
+
+
+def test_graph_replays_of_many_rows_match_eager():
+    """The calls of many rows captured in one graph: every replay gives the eager bits."""
+    need_gpu()
+    from gpu_util import dev, host, torch
+    from moa_amd import ops
+    ops.init(0)
+    up = lambda d, *skip: {k: dev(v) for k, v in d.items() if isinstance(v, np.ndarray) and k not in skip}
+    i32 = lambda v: torch.tensor([int(v)], dtype=torch.int32, device="cuda")
+    bits = lambda *shape: torch.zeros(shape, dtype=torch.int16, device="cuda")
+    f32 = lambda n: torch.zeros(n, device="cuda")
+    at = up(synth.cfg_attention(9, M=40, pos=300 + np.arange(40)))
+    qv = synth.cfg_qkv(9, M=40, pos=1000)
+    Q, ffn, o = up(qv), up(synth.cfg_ffn_fp8(9, M=40)), up(synth.cfg_o(9, M=40))
+    fq = synth.cfg_full_qkv(9, M=20, pos=30)
+    F, fo = up(fq), up(synth.cfg_full_o(9, M=20))
+    fa, pg = up(synth.cfg_full_attention(9, M=66, P=2, q_std=0.3)), up(synth.cfg_full_attention(8, M=19, P=2, q_std=0.3))
+    lg, lm = up(synth.cfg_logits(9, M=24)), synth.lm_head_device(9)
+    kv, ro, fkv, fro = i32(qv["kv_offset"]), i32(qv["rope_offset"]), i32(fq["kv_offset"]), i32(fq["rope_offset"])
+    outs = dict(attn=bits(40, 4096), q=bits(40, 4096), kc=bits(*Q["k_cache"].shape), vc=bits(*Q["v_cache"].shape),
+                res=bits(40, 3840), fq=bits(20, 8192), fk=bits(*F["k_cache"].shape), fv=bits(*F["v_cache"].shape),
+                fres=bits(20, 3840), fmax=f32(66 * 16), fsum=f32(66 * 16), fout=bits(66, 8192), pmax=f32(19 * 16),
+                psum=f32(19 * 16), pout=bits(19, 8192), logits=bits(24, synth.W))
+    t = outs
+
+    def step():
+        for n, x in (("kc", Q["k_cache"]), ("vc", Q["v_cache"]), ("res", o["residual"]), ("fk", F["k_cache"]),
+                     ("fv", F["v_cache"]), ("fres", fo["residual"])):
+            t[n].copy_(x)
+        ops.sliding_attention(at["q"], at["k_cache"], at["v_cache"], at["mask"], t["attn"])
+        ops.sliding_project_qkv(Q["x"], Q["q_weight"], Q["k_weight"], Q["v_weight"], Q["q_weight_scale"],
+                                Q["k_weight_scale"], Q["v_weight_scale"], Q["input_rms_weight"], Q["q_rms_weight"],
+                                Q["k_rms_weight"], kv, ro, Q["cos"], Q["sin"], t["kc"], t["vc"], t["q"])
+        ops.sliding_attention_output_feedforward_fp8(
+            o["x"], o["post_attn_rms_weight"], o["o_weight"], o["o_weight_scale"], t["res"], ffn["pre_ff_rms_weight"],
+            ffn["up_weight"], ffn["gate_weight"], ffn["down_weight"], ffn["up_weight_scale"], ffn["gate_weight_scale"],
+            ffn["down_weight_scale"], ffn["post_ff_rms_weight"], ffn["layer_scalar"])
+        ops.full_project_qkv(F["x"], F["q_weight"], F["k_weight"], F["q_weight_scale"], F["k_weight_scale"],
+                             F["input_rms_weight"], F["q_rms_weight"], F["k_rms_weight"], fkv, fro, F["cos"], F["sin"],
+                             t["fk"], t["fv"], t["fq"])
+        ops.full_attention_output(fo["x"], fo["running_sum"], fo["post_attn_rms_weight"], fo["o_weight"],
+                                  fo["o_weight_scale"], t["fres"])
+        ops.full_attention(fa["q"], fa["k_pages"], fa["v_pages"], fa["masks"], t["fmax"], t["fsum"], t["fout"])
+        for p, call in enumerate((ops.full_attention_first_page, ops.full_attention_page)):
+            call(pg["q"], pg["k_pages"][p], pg["v_pages"][p], pg["masks"][p], t["pmax"], t["psum"], t["pout"])
+        ops.final_norm_and_logits(lg["input"], lg["rms_weight"], lm, t["logits"])
+
+    def read():
+        return {n: host(x).copy() for n, x in t.items()}
+
+    step()
+    want = read()
+    assert ops.device_errors() == 0 and all(w.any() for w in want.values())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        step()
+    for replay in range(4):
+        say(f"graph replay {replay}")
+        for x in t.values():
+            x.fill_(0)  # eager work between replays
+        torch.cuda.synchronize()
+        g.replay()
+        for n, got in read().items():
+            assert np.array_equal(want[n], got), f"replay {replay}: {n} differs from the eager result"
+        step()
+        for n, got in read().items():
+            assert np.array_equal(want[n], got), f"eager after replay {replay}: {n}"
+    assert ops.device_errors() == 0
