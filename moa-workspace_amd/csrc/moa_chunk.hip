@@ -12,7 +12,12 @@
 //   FFN: RMSNorm rows -> up and gate GEMMs in one kernel with the GeGLU epilogue -> down GEMM
 //        (split-K) -> post-RMSNorm + residual + layer scalar
 // Rounding points are those of the oracle (FO/scripts/generate_references.py:265-274, 337-414;
-// FO/scripts/reference/gemma4.py:83-89, 189-197); only the f32 accumulation order differs.
+// FO/scripts/reference/gemma4.py:83-89, 189-197); only the f32 accumulation order differs. It depends on the
+// row count: up to 64 rows the tiles of 128 weight rows (FFN, full-attention QKV) add two k groups, and the k splits
+// change at 129 (QKV), 257 and 513 rows, so a row's last bits may differ between calls of different sizes.
+//
+// The figures in the comments below compare variants in turn on one MI355X; between comments the card may be
+// another (the FP8 layer of 1000 rows takes 437-484 us across cards and stages of this file).
 #include <hip/hip_runtime.h>
 
 #include "moa_device.h"
@@ -279,8 +284,8 @@ void chunk_gemm_kernel(GemmArgs g) {
     __syncthreads();
     read_b(bb[0], 0, 0);
     // With 128 weight rows the weights are requested two steps at a time (in odd steps), so that both halves of a
-    // 128-byte line go out together: GeGLU of 17 rows 30.8 -> 28.4 us, FP8 layer of 17 rows 88.5 -> 85.7, of 1000
-    // rows 470 -> 464, NVFP4 494 -> 489. With 64 (O, QKV) the second load only holds the step up: 10.9 -> 11.9 us.
+    // 128-byte line go out together: GeGLU of 17 rows 30.8 -> 28.4 us; FP8 layer of 64 rows 79 -> 77, of 128 rows
+    // 110.5 -> 108.5, of 1000 rows 468 -> 464, NVFP4 488 -> 481. With 64 (O, QKV) the second load only holds the step up: 10.9 -> 11.9 us.
     auto next_w = [&](auto P, int s) {
         constexpr int c = decltype(P)::value;
         if constexpr (BN == 64) {

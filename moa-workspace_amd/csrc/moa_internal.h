@@ -55,7 +55,9 @@ constexpr int kFaDimBlocks = 4;
 constexpr int kFaRec = 2 * kGf + kGf * kDf;
 constexpr int kFaMaxRecords = 256;                        // records per row of the fused pass
 constexpr int kFaSplitPages = 8;                           // the fused pass splits dims up to 8 pages
-constexpr int kFattnRecords = 1024;                        // records of scratch (>= kMaxDecodeM * kFaChunks)
+// Records of scratch, 32.9 KB each: 33.7 MB per device. Enough for four rows of 256 records, one launch of the rows
+// kernel on four rows (256 records, 8.4 MB, hold one row).
+constexpr int kFattnRecords = 1024;                        // >= kMaxDecodeM * kFaChunks
 constexpr size_t kFattnPartFloats = (size_t)kFattnRecords * kFaRec;
 
 // Tagged hand-off words of the single-launch FFN (per workgroup a partial sum, 8 output words and

@@ -25,7 +25,7 @@ constexpr int kLmBlock = kWave * kLmSlices;
 constexpr int kLmK = kH / kLmSlices;     // k of each
 constexpr int kLmPairs = kLmK / 64;      // 128-byte lines of a vocabulary row in it (two MFMA k steps each)
 constexpr int kLmTileBytes = 16 * kH * (int)sizeof(uint16_t);
-constexpr int kLmNt = 2;                 // cache policy of the stream: non-temporal (default: 342 against 299 us, 16 rows)
+constexpr int kLmNt = 2;                 // cache policy of the stream: non-temporal (default: 341 against 296 us, 16 rows)
 static_assert(kLmK % 64 == 0, "whole lines per slice");
 
 // LDS barrier that leaves global loads in flight.
@@ -39,7 +39,7 @@ __device__ __forceinline__ void lm_barrier() {
 // 4: lane (r, g) = (lane % 16, lane / 16) holds chunk 2 g + r / 8 (16 bytes) of row r % 8 in a and of
 // row 8 + r % 8 in b. One exchange between lanes r and r ^ 8 (DPP) gives every lane its own row r:
 // f[0] chunk 2 g, f[1] chunk 2 g + 1. (Loads in the MFMA's layout move 64 bytes of 16 rows each, half
-// a line per request: 347 us at 2 rows against 308 so, and no faster with twice the bytes in flight.)
+// a line per request: 460 us at one row against 291 so, 387 against 290 at 2, 396 against 299 at 24.)
 __device__ __forceinline__ void lm_rows(const uint4& a, const uint4& b, bf16x8 (&f)[2]) {
     const uint32_t av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
     uint32_t x[4], y[4];
@@ -76,10 +76,10 @@ __device__ __forceinline__ uint4 lm_scale(const uint4& x, float inv, const float
 // per CU. Each wave has five pairs of loads in flight, 120 KB (240 KB) per CU. The logits wait in
 // LDS and go out at the end, 2 KB per token: written 32 or 128 bytes at a time between the reads,
 // 16 rows' logits (8 MB) cost 20 us.
-// Measured (2.01 GB; the box's attainable read rate takes 285 us): one row 291 us (on eight lanes per
-// vocabulary row and v_dot2, 16 waves per CU: 294), 2 rows 296, 16 rows 299 (1667 that way), 24 rows
-// 312 (2640). What the rows over 1 still pay is waves waiting at the meetings: 16-row meetings take 307
-// us at 2 rows and 320 at 24. Whole vocabulary rows per wave against token rows in LDS have no
+// Measured (2.01 GB; the card's attainable read rate takes 285 us): one row 289-292 us by card (on eight lanes
+// per vocabulary row and v_dot2, 16 waves per CU: 294), 2 rows 290-294, 16 rows 292-296 (1667 that way), 24 rows
+// 300-311 (2640). What the rows over 16 still pay is waves waiting at the meetings: with VT = 1 one row takes
+// 297 us against 289, 2 rows 313 against 294, 16 rows 318 against 296, 24 rows 321 against 310. Whole vocabulary rows per wave against token rows in LDS have no
 // meetings, but a CU then reads from 256 rows at once: 326 us at one row.
 template <int MT, int VT, bool DB, bool One = false>
 __global__ __launch_bounds__(kLmBlock, One ? 6 : 3) void logits_kernel(const uint16_t* __restrict__ input,
