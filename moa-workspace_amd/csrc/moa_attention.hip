@@ -250,8 +250,8 @@ constexpr int kArMaxBlocks = 32;                // row blocks x slot parts of a 
 // Weights are exp(score - reference) with a reference at most this far below the row's largest score: out
 // (128 accumulators a lane) is rescaled only when the maximum has grown by more.
 constexpr float kArSlack = 8.0f;
-constexpr int kArMinRows = 6;                   // rows of a call from which this path is used: 12 us up to 16 rows, a
-                                                // workgroup set per row takes 11.7 us at 5 rows, 12.1 at 6, 14.2 at 8
+constexpr int kArMinRows = 6;                   // rows of a call from which this path is used. 6 rows 11.3 us (window just begun) to
+                                                // 12.1 (full), 7 rows 11.8-12.4; a workgroup set per row 11.8, 12.7
 static_assert((size_t)kNs * kArMaxBlocks * kArQ * kArRec <= kAttnPartFloats, "records fit the scratch");
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
